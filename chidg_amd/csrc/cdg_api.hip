@@ -782,11 +782,27 @@ extern "C" int cdg_prec_create(cdg_ctx *ctx, const cdg_mat *A, int32_t type, int
     M->part_cap = part_doubles;
     if (!e && M->apply_mode == CDG_APPLY_DATAFLOW) e = df_setup(ctx, M);
     if (!e && M->apply_mode == CDG_APPLY_FOLDED) e = alloc(&M->W, es * (size_t)M->nup * M->ld);
-    if (!e) {   // the single-vector sweep's plan, so that an apply never allocates
+    if (const char *f = std::getenv("CDG_FOLD_AFTER")) M->fold_after = std::max(0, std::atoi(f));
+    if (!e) {   // the single-vector sweep's plans and W, so that an apply never allocates
         SweepPlan *p = nullptr;
-        const int es = sweep_plan(ctx, M, 1, 0, M->nrows, &p);
-        if (es == CDG_ERR_UNSUPPORTED) M->sweep_ok = 0;
-        else e = es;
+        int ep = sweep_plan(ctx, M, 1, 0, M->nrows, false, &p);
+        if (ep == CDG_ERR_UNSUPPORTED) M->sweep_ok = 0;
+        else e = ep;
+        if (!e && M->sweep_ok && precision == CDG_BF16 && M->nup > 0 && M->maxdep <= 6) {
+            ep = sweep_plan(ctx, M, 1, 0, M->nrows, true, &p);
+            if (!ep) {
+                std::vector<int32_t> up_row(M->nup);
+                for (int i = 0; i < M->nrows; ++i)
+                    for (int u = S->up_ptr[i]; u < S->up_ptr[i + 1]; ++u) up_row[u] = i;
+                M->fold_ok = 1;
+                e = alloc(&M->W, es * (size_t)M->nup * M->ld);
+                if (!e) e = upload_array(ctx, &M->d_up_row, up_row, &M->owned);
+                if (!e && hipStreamSynchronize(ctx->stream) != hipSuccess)   // up_row is host memory
+                    e = cdg_fail(ctx, CDG_ERR_HIP, "upload of the upper entries' rows");
+            } else if (ep != CDG_ERR_UNSUPPORTED) {
+                e = ep;
+            }
+        }
     }
     if (!e) {
         hipError_t he = hipStreamSynchronize(ctx->stream);
@@ -1023,11 +1039,45 @@ extern "C" int cdg_prec_update(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, int3
     if (M->type == CDG_PREC_IDENTITY) { M->stamp = A->stamp; M->factored = 1; return CDG_OK; }
     M->factored = 0;
     M->w_ready = 0;
+    M->w_asked = 0;
+    M->prev_napply = M->napply;
+    M->napply = 0;
     int e = launch_ilu_factor(ctx, M, A, bad_row);
     if (e) return e;
     M->stamp = A->stamp;
     M->factored = 1;
-    return CDG_OK;
+    return M->w_keep ? sweep_fold(ctx, M, A) : CDG_OK;
+}
+
+// W of the current factor, formed once per factor (kernels only).  Under capture the launch that
+// forms it belongs to the graph: it has not run yet, so the next eager apply forms W itself; and
+// as a captured apply may also read a W that is there already, updates form it from then on.
+int sweep_fold(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    CDG_HIP_TRY(hipStreamIsCapturing(ctx->stream, &cap));
+    const bool captured = cap != hipStreamCaptureStatusNone;
+    if (captured) M->w_keep = 1;
+    if (M->w_ready) return CDG_OK;
+    int e = launch_fold_left(ctx, M, A);
+    if (!e && !captured) M->w_ready = 1;
+    return e;
+}
+
+// The sweep for k vectors, in the form that M's schedule and history ask for.  Several vectors and
+// the schedules STREAM and ROWSLICE take W where there is one.
+static int prec_sweep(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t len, int k) {
+    bool fold = false;
+    if (M->fold_ok) {
+        M->napply += k;
+        if (k > 1 || M->apply_mode == CDG_APPLY_STREAM || M->apply_mode == CDG_APPLY_ROWSLICE) M->w_asked = 1, fold = true;
+        else if (M->apply_mode == CDG_APPLY_AUTO)
+            fold = M->w_asked || (M->fold_after > 0 && (M->napply > M->fold_after || M->prev_napply > M->fold_after));
+        if (fold) {
+            int e = sweep_fold(ctx, M, A);
+            if (e) return e;
+        }
+    }
+    return launch_ilu_sweep(ctx, M, A, v, z, len, k, fold);
 }
 
 static int prec_apply_dev(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z) {
@@ -1037,7 +1087,7 @@ static int prec_apply_dev(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const dou
     if (M->apply_mode == CDG_APPLY_DATAFLOW) return launch_ilu_apply_df(ctx, M, A, v, z);
     // one persistent sweep for every schedule but FOLDED; patterns it does not
     // take (more blocks in a row than a task record holds) use level launches
-    if (M->apply_mode != CDG_APPLY_FOLDED && M->sweep_ok) return launch_ilu_sweep(ctx, M, A, v, z, len, 1);
+    if (M->apply_mode != CDG_APPLY_FOLDED && M->sweep_ok) return prec_sweep(ctx, M, A, v, z, len, 1);
     const bool fold_now = !M->w_ready && M->apply_mode == CDG_APPLY_FOLDED;   // schedule chosen after the factor
     if (fold_now) {
         if (!M->W) {
@@ -1224,7 +1274,7 @@ int fetch_small(cdg_ctx *ctx, size_t n) {
 int prec_apply_multi(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t len, int k) {
     if (M->type == CDG_PREC_IDENTITY) return kv_copy(ctx, len * k, v, z);
     if (!M->factored) return cdg_fail(ctx, CDG_ERR_STATE, "ILU0 apply before update");
-    if (k > 1 && M->sweep_ok) return launch_ilu_sweep(ctx, M, A, v, z, len, k);
+    if (k > 1 && M->sweep_ok) return prec_sweep(ctx, M, A, v, z, len, k);
     for (int r = 0; r < k; ++r) {
         int e = prec_apply_dev(ctx, M, A, v + (size_t)r * len, z + (size_t)r * len);
         if (e) return e;
@@ -1330,6 +1380,12 @@ int fgmres_lanes(Solver &S, std::vector<Level> &lvs, int depth, int k, const dou
             if (e) return e;
         }
         e = see(seqs.size());
+        if (!e && S.M->fold_ok) {   // applies that were queued after every lane had stopped did not happen
+            int steps = 0;
+            for (int r = 0; r < k; ++r)
+                if (!done[r]) steps = std::max(steps, (int)((uint32_t)res[r].word >> ARN_W_BITS));
+            S.M->napply -= k * ((int)seqs.size() - 1 - steps);
+        }
         // x = x0 + Z y   (:287-295); stopped lanes are done, the others restart
         if (!e) e = arn_cycle_end(ctx, lv.arn, lv.Z, X, lv.x0, first);
         if (e) return e;

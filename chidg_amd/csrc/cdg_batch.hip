@@ -371,7 +371,8 @@ int batch_step(cdg_ctx *ctx, cdg_batch *bt, int j, double tol, double rtol, int 
         hipLaunchKernelGGL(k_browk, dim3((g.U->nrows + 255) / 256), dim3(256), 0, ctx->stream, g.U->nrows, g.d_row_sys,
                            bt->d_sys_lane0, bt->d_sys_nrhs, bt->st.active, g.d_row_kl);
         for (const auto &r : g.ap_ranges) {
-            int e = launch_ilu_sweep(ctx, g.M, g.U, Vj + g.goff, Zj + g.goff, bt->Ltot, r[2], g.d_row_kl, r[0], r[1]);
+            int e = launch_ilu_sweep(ctx, g.M, g.U, Vj + g.goff, Zj + g.goff, bt->Ltot, r[2], g.M->fold_ok != 0, g.d_row_kl,
+                                     r[0], r[1]);
             if (e) return e;
         }
         int e = group_mv(ctx, bt, g, Zj, W, g.d_row_kl);
@@ -613,8 +614,9 @@ extern "C" int cdg_batch_create(cdg_ctx *ctx, int32_t nsys, cdg_mat *const *A, c
         const double tf = bsecs(tg);
         for (const auto &r : g.ap_ranges) {   // the sweeps' plans (nothing is allocated later)
             SweepPlan *p = nullptr;
-            if (!e) e = sweep_plan(ctx, g.M, r[2], r[0], r[1], &p);
+            if (!e) e = sweep_plan(ctx, g.M, r[2], r[0], r[1], g.M->fold_ok != 0, &p);
         }
+        if (!e && g.M->fold_ok) e = sweep_fold(ctx, g.M, g.U);
         if (btrace())
             std::fprintf(stderr, "[batch] group n=%d: %d systems, %d rows, factor %.3f s, sweep plans %.3f s\n", g.n,
                          (int)g.members.size(), g.U ? g.U->nrows : 0, tf, bsecs(tg) - tf);
@@ -652,6 +654,7 @@ extern "C" int cdg_batch_update(cdg_ctx *ctx, cdg_batch *bt, cdg_mat *const *A) 
             b0 += A[s]->nnzb;
         }
         if (!e) e = cdg_prec_update(ctx, g.M, g.U, nullptr);
+        if (!e && g.M->fold_ok) e = sweep_fold(ctx, g.M, g.U);
     }
     if (!e) CDG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     if (btrace()) std::fprintf(stderr, "[batch] update: copies and factors %.3f s\n", bsecs(t0));

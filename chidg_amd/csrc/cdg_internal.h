@@ -85,7 +85,8 @@ struct SweepShape {
 // order, exchange words and ticket counter (device memory of the preconditioner).
 struct SweepPlan {
     SweepShape sh;
-    int KT = 1, lo = 0, hi = 0, G = 1, nunits = 0, grid = 0, spin = 0;
+    int KT = 1, lo = 0, hi = 0, G = 1, nunits = 0, grid = 0, spin = 0, dep = 1;
+    bool fold = false;            // over W = Dinv U
     size_t lds = 0;
     const void *fn = nullptr;
     int32_t *recs = nullptr;
@@ -122,10 +123,12 @@ struct cdg_prec {
     void *U = nullptr;                 // nup slots (FP32/BF16 copies of A's upper blocks)
     // nup slots, FP64/FP32: W_u = A_{up_blk[u]} Dinv_{up_col[u]}, the upper
     // blocks with the Dinv of their column folded in (the level schedule's
-    // backward sweep is then one stage per level); null for BF16
+    // backward sweep is then one stage per level).  BF16: W_u = Dinv_{row(u)} A_{up_blk[u]}, of the
+    // sweep's folded form (fold_ok)
     void *W = nullptr;
     int32_t w_ready = 0;               // W holds the current factor's products
     int32_t *d_up_all = nullptr;       // 0..nup-1 (the W jobs)
+    int32_t *d_up_row = nullptr;       // row of each upper entry (fold_ok)
     void *Dinv = nullptr;              // nrows slots
     float *L32 = nullptr, *D32 = nullptr;   // FP32 work for the BF16 variant
     void *inv_w = nullptr;             // working slots of the global-memory block inverse
@@ -169,9 +172,15 @@ struct cdg_prec {
     int32_t df_spin = 1 << 21;         // polls before a dependency wait gives up
     // the sweep (k_sweep.hip): plans made so far (row range, right-hand sides)
     std::vector<SweepPlan *> sweeps;
-    SweepShape sweep_sh;
-    int32_t sweep_shaped = 0;
+    SweepShape sweep_sh[2];            // plain, and over W
+    int32_t sweep_shaped[2] = {0, 0};
     int32_t sweep_ok = 1;              // 0: the pattern does not fit the sweep (level launches instead)
+    // BF16, where a row's upper blocks and its Dinv fit a task: the sweep over W = Dinv U.  CDG_APPLY_AUTO
+    // takes it once the factor has served fold_after applies (0: never), from the first apply when the
+    // previous factor served more, or when another call has formed W for this factor.
+    int32_t fold_ok = 0, fold_after = 12, napply = 0, prev_napply = 0;
+    int32_t w_asked = 0;               // W of this factor was asked for by name or for several vectors
+    int32_t w_keep = 0;                // a captured launch reads W: every update forms it anew
     int32_t noalloc_ok = 0;            // CDG_SCHEDULE_ROWSLICE or _STREAM was set (cdg_prec_apply_noalloc)
     uint64_t stamp = 0;
     int32_t factored = 0;
@@ -183,8 +192,9 @@ enum { ARN_CGS = 0, ARN_MGS = 1, ARN_START = 2, ARN_NORM = 3 };
 enum { ARN_ACTIVE, ARN_DONE, ARN_NVECS, ARN_NITER, ARN_CONV, ARN_NREORTH, ARN_SECOND, ARN_RUN, ARN_NST = 32 };   // int state of a lane (a line)
 enum { ARN_R0INIT, ARN_RES, ARN_TP, ARN_TM, ARN_TO, ARN_TN, ARN_NSC = 16 };                 // doubles of a lane
 // What launches report per lane, in pinned memory: after each step one word, the
-// launch's number and ARN_W_* bits; the rest with the word of an ARN_NORM launch.
-enum { ARN_W_ACTIVE = 1, ARN_W_DONE = 2, ARN_W_ERR = 4 };
+// launch's number, the lane's steps in this cycle and ARN_W_* bits; the rest with the word of an
+// ARN_NORM launch.
+enum { ARN_W_ACTIVE = 1, ARN_W_DONE = 2, ARN_W_ERR = 4, ARN_W_BITS = 3 };
 struct ArnRes {
     uint64_t word;
     double res, t[4];             // ||b - A x||; ticks: preconditioner, product, vectors, norms
@@ -229,10 +239,12 @@ enum { CDG_APPLY_LEVELS = 0, CDG_APPLY_DATAFLOW = 1, CDG_APPLY_FOLDED = 2, CDG_A
        CDG_APPLY_ROWSLICE = 5 };
 // the sweep (k_sweep.hip)
 bool sweep_shape(int n, int precision, int maxdep, int width, int cus, SweepShape *out);
-int sweep_plan(cdg_ctx *ctx, cdg_prec *M, int K, int lo, int hi, SweepPlan **out);
+int sweep_plan(cdg_ctx *ctx, cdg_prec *M, int K, int lo, int hi, bool fold, SweepPlan **out);
+int sweep_fold(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A);
 void sweep_free(cdg_prec *M);
 int launch_ilu_sweep(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t stride, int k,
-                     const int32_t *row_k = nullptr, int lo = 0, int hi = -1);
+                     bool fold, const int32_t *row_k = nullptr, int lo = 0, int hi = -1);
+int launch_fold_left(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A);
 int launch_mv_multi(cdg_ctx *ctx, const cdg_mat *A, const double *X, double *Y, int64_t stride, int k,
                     const int32_t *row_k = nullptr, int row_lo = 0, int row_hi = -1);
 bool is_device_ptr(const void *p);

@@ -24,5 +24,10 @@ extern "C" int cdg_prec_apply_noalloc(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *
     if (!M->factored) return cdg_fail(ctx, CDG_ERR_STATE, "ILU0 apply before update");
     if (!M->noalloc_ok)
         return cdg_fail(ctx, CDG_ERR_STATE, "cdg_prec_apply_noalloc: set CDG_SCHEDULE_ROWSLICE or CDG_SCHEDULE_STREAM first");
-    return launch_ilu_sweep(ctx, M, A, v, z, (int64_t)M->nrows * M->n, 1);
+    if (M->fold_ok) {   // W is there; the first call after an update forms its values
+        M->w_asked = 1;
+        int e = sweep_fold(ctx, M, A);
+        if (e) return e;
+    }
+    return launch_ilu_sweep(ctx, M, A, v, z, (int64_t)M->nrows * M->n, 1, M->fold_ok != 0);
 }

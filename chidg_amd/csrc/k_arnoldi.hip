@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(256) k_arn_finish(ArnArgs a) {
     if (!runs) {
         if (blockIdx.x == 0 && tid == 0) {                  // say again how the lane ended
             const double res = sc[ARN_RES];
-            uint64_t word = (uint64_t)a.seq << 32 | (isfinite(res) ? 0 : ARN_W_ERR);
+            uint64_t word = (uint64_t)a.seq << 32 | (uint64_t)(uint32_t)st[ARN_NVECS] << ARN_W_BITS | (isfinite(res) ? 0 : ARN_W_ERR);
             if (st[ARN_CONV] || !(res > a.tol)) word |= ARN_W_DONE;
             put(&a.hres[l].word, word);
         }
@@ -385,7 +385,8 @@ __global__ void __launch_bounds__(256) k_arn_finish(ArnArgs a) {
             sc[ARN_TN] += (double)(now - a.stamp[2]);
         }
         ArnRes *const o = a.hres + l;
-        uint64_t word = (uint64_t)a.seq << 32 | (active ? ARN_W_ACTIVE : 0) | (err ? ARN_W_ERR : 0);
+        uint64_t word = (uint64_t)a.seq << 32 | (uint64_t)(steps ? jj : 0) << ARN_W_BITS | (active ? ARN_W_ACTIVE : 0) |
+                        (err ? ARN_W_ERR : 0);
         if (conv || !(res > a.tol)) word |= ARN_W_DONE;
         if (a.mode == ARN_NORM) {                       // the report of the whole solve
             put(&o->res, res);

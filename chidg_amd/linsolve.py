@@ -264,8 +264,10 @@ class _Preconditioner:
 
     def set_schedule(self, schedule: str):
         """ILU(0) apply schedule: 'auto' (the default), 'levels', 'stream' and
-        'rowslice' run one persistent sweep over tasks of (row, column chunk),
-        the same bits under all four names; 'dataflow' is a persistent launch
+        'rowslice' run one persistent sweep over tasks of (row, column chunk):
+        in FP64 and FP32 the same bits under all four names, in BF16 'stream' and
+        'rowslice' with W = Dinv U rounded once from the FP32 Dinv, 'auto' from
+        the 13th apply of a factor on; 'dataflow' is a persistent launch
         over column slices with partial sums, 'folded' one launch per wavefront
         level with Dinv folded into the upper blocks at the first apply after
         each factor (FP64/FP32)."""

@@ -168,27 +168,35 @@ int cdg_prec_update(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, int32_t *bad_ro
 int cdg_prec_apply(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z);
 int cdg_prec_apply_async(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z);
 /* Z_r = M^-1 V_r for r < k (k vectors one after another, host or device):
- * one sweep for up to 8 vectors at once (ILU(0)); each Z_r has the bits of the
- * default schedule's apply of V_r alone.
+ * one sweep for up to 8 vectors at once (ILU(0)); each Z_r has the bits of
+ * CDG_SCHEDULE_ROWSLICE's apply of V_r alone.
  * precon_ILU0%apply (precon_ILU0.f90:286-411) per vector in the reference. */
 int cdg_prec_apply_multi(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, int32_t k, const double *V, double *Z);
 /* preconditioner%tear_down (precon_ILU0.f90:450-470). */
 int cdg_prec_destroy(cdg_ctx *ctx, cdg_prec *M);
 /* Schedule of the ILU(0) apply (no reference counterpart: the reference's
  * apply is one sequential loop over rows, precon_ILU0.f90:286-411).  All give
- * the same result to rounding:
+ * the same result to the rounding of the factor's storage:
  *   CDG_SCHEDULE_AUTO      (the default), CDG_SCHEDULE_LEVELS,
  *   CDG_SCHEDULE_STREAM, CDG_SCHEDULE_ROWSLICE
  *                          one persistent launch over tasks of (row, column
  *                          chunk) that read the factor as it is stored and
- *                          pass values from task to task: one kernel, the same
- *                          bits under all four names.  Nothing is prepared
- *                          per factor and no call allocates, so a call may be
- *                          captured in a graph and replayed.  STREAM and
- *                          ROWSLICE are refused (CDG_ERR_UNSUPPORTED) for rows
- *                          of more than 6 lower or upper blocks; AUTO and
- *                          LEVELS use one launch per wavefront level for
- *                          rows of more than 7.
+ *                          pass values from task to task.  No call allocates,
+ *                          so a call may be captured in a graph and replayed.
+ *                          FP64 and FP32: one kernel, the same bits under all
+ *                          four names, nothing prepared per factor.  BF16:
+ *                          LEVELS applies L, U and Dinv as stored; STREAM and
+ *                          ROWSLICE (and several vectors at once) apply L, Dinv
+ *                          and W = Dinv U, which the first such call after each
+ *                          factor forms from the FP32 Dinv and rounds once;
+ *                          AUTO goes from the first to the second at the 13th
+ *                          apply after a factor, or at the first when the
+ *                          previous factor served more than 12 (environment
+ *                          CDG_FOLD_AFTER=k sets k; 0 never) or another call
+ *                          has formed W.  STREAM and ROWSLICE are refused
+ *                          (CDG_ERR_UNSUPPORTED) for rows of more than 6
+ *                          lower or upper blocks; AUTO and LEVELS use one
+ *                          launch per wavefront level for rows of more than 7.
  *   CDG_SCHEDULE_DATAFLOW  one persistent launch over column slices with
  *                          completion counters
  *   CDG_SCHEDULE_FOLDED    one launch per wavefront level with Dinv folded into
