@@ -740,6 +740,151 @@ __device__ __forceinline__ bool panel_steps(T *G, int gp, int NP, int n, int k0,
     return __builtin_amdgcn_readfirstlane(*miss_sh) != 0;
 }
 
+// The panel of BF16-stored factors (FP32): the same Gauss-Jordan, rounded step by step as an unblocked
+// one rounds.  A factor in BF16 is read through its 8 bits: where FP32 rounds the other way, one
+// entry in 20000 lands on the next BF16 value, which moves the apply by 4e-5 and a solve's residual
+// norm by 1e-4 of itself.  So this storage keeps one order of operations: each step's pivot row is scaled by
+// 1 / pivot and subtracted, by every row, before the next step.
+//   Stage A (wavefront 0): the pivot block as in panel_steps; each step's scaled pivot row (1 / pivot
+//   in its own column) and the pivot itself go to H[j] (zeros for steps from w on), then *step_sh rises to
+//   k0 + j + 1.
+//   Stage B (wavefronts 1..NW-1, a row per lane) replays step j once *step_sh shows it.  Wavefront 0
+//   never waits, so every wait ends; k0 only grows during a kernel, *step_sh starts at 0.
+// G, the checks and the result as in panel_steps.  Whole BF16 factors with it and with panel_steps:
+// 16^3 P2 7.4 and 6.9 ms, 16^3 P3 37.2 and 34.4, 31x17x13 P1 1.84 and 1.53.
+constexpr int kHP = 20;   // pitch of H: 16 values and the pivot, 16-byte rows
+template <int NW>
+__device__ __forceinline__ bool panel_replay(float *G, int gp, int NP, int n, int k0, int w, float (*H)[kHP],
+                                             int32_t *step_sh, int32_t *miss_sh) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    bool viol = false;
+    if (tid < 64) {
+        const int i = lane & 15, q = lane >> 4;
+        float a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = G[(k0 + i) * gp + 4 * q + e];
+        unrolled<0, 16>([&](auto jc) {
+            constexpr int j = decltype(jc)::value, jq = j >> 2, je = j & 3;
+            const bool isp = i == j, mine = q == jq;
+            float sv[4] = {0.f, 0.f, 0.f, 0.f}, piv = 0.f;
+            if (j < w) {
+                piv = readlane(a[je], 16 * jq + j);
+                const float rinv = recip(piv), ap = fabsf(piv), cc = row_all<jq>(a[je]);
+                viol = viol || !(ap > 0.f) || !(ap < INFINITY) || (i > j && k0 + i < n && (float)kPivTau * fabsf(cc) > ap);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sv[e] = newbcast<j>(a[e]) * rinv;
+                    if (e == je) sv[e] = mine ? rinv : sv[e];
+                    const float t = isp ? sv[e] : fmaf(-cc, sv[e], a[e]);
+                    a[e] = e == je && mine ? (isp ? rinv : -cc * rinv) : t;
+                }
+            }
+            if (i == 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) H[j][4 * q + e] = sv[e];
+                if (q == 0) H[j][16] = piv;
+            }
+            if (tid == 0) __hip_atomic_store(step_sh, k0 + j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        });
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = 4 * q + e;
+            G[(k0 + i) * gp + c] = a[e] - (i == c && c < w ? 1.f : 0.f);
+        }
+    } else {
+        const int row = lane * (NW - 1) + (tid >> 6) - 1;
+        const bool live = row < NP && (row < k0 || row >= k0 + 16), unused = row >= k0 + 16 && row < n;
+        float pr[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) pr[c] = live ? G[row * gp + c] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            while (__hip_atomic_load(step_sh, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <= k0 + j)
+                __builtin_amdgcn_s_sleep(1);
+            float sv[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) sv[c] = H[j][c];
+            const float cc = pr[j];
+            viol = viol || (j < w && unused && (float)kPivTau * fabsf(cc) > fabsf(H[j][16]));
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+                if (c != j) pr[c] = fmaf(-cc, sv[c], pr[c]);
+            pr[j] = -cc * sv[j];
+        }
+        if (live)
+#pragma unroll
+            for (int c = 0; c < 16; ++c) G[row * gp + c] = pr[c];
+    }
+    if (viol) *miss_sh = 1;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*miss_sh) != 0;
+}
+
+// The same steps spread over a workgroup of 16 wavefronts (128 VGPRs a lane leave no room for stage
+// A beside stage B): row r in lane r, one barrier a step.  The owner of the pivot row publishes it, scaled,
+// and the pivot's size in H[j % 2].
+template <int NW>
+__device__ __forceinline__ bool panel_rows(float *G, int gp, int NP, int n, int k0, int w, float (*H)[kHP],
+                                           int32_t *miss_sh) {
+    const int row = threadIdx.x;
+    const bool live = row < NP, wave_live = __builtin_amdgcn_readfirstlane(row & ~63) < NP;
+    float pr[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) pr[c] = live ? G[row * gp + c] : 0.f;
+    bool used = row >= n || row < k0, viol = false;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        if (j < w) {
+            float *const h = H[j & 1];
+            const bool isp = row == k0 + j;
+            if (isp) {
+                const float ap = fabsf(pr[j]), rinv = 1.f / pr[j];
+                viol = viol || !(ap > 0.f) || !(ap < INFINITY);
+#pragma unroll
+                for (int c = 0; c < 16; ++c) h[c] = pr[c] = c == j ? rinv : pr[c] * rinv;
+                h[16] = ap;
+            }
+            __syncthreads();   // (the next step writes the other half of H)
+            if (wave_live && !isp) {
+                float sv[17];
+#pragma unroll
+                for (int c = 0; c < 17; ++c) sv[c] = h[c];
+                const float cc = pr[j];
+                viol = viol || (!used && (float)kPivTau * fabsf(cc) > sv[16]);
+#pragma unroll
+                for (int c = 0; c < 16; ++c) pr[c] = c == j ? -cc * sv[j] : fmaf(-cc, sv[c], pr[c]);
+            }
+            used = used || isp;
+        }
+    }
+    if (live)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) G[row * gp + c] = pr[c] - (row - k0 == c && c < w ? 1.f : 0.f);
+    if (viol) *miss_sh = 1;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*miss_sh) != 0;
+}
+
+// LDS of a panel's steps, and the steps: REPLAY for BF16-stored factors.
+template <typename T, bool REPLAY> struct PanelLds {
+    T Ws[16][17], Ls[16][17];
+    __device__ __forceinline__ void start() {}
+    template <int NW>
+    __device__ __forceinline__ bool run(T *G, int gp, int NP, int n, int k0, int w, int32_t *miss_sh) {
+        return panel_steps<T, NW>(G, gp, NP, n, k0, w, Ws, Ls, miss_sh);
+    }
+};
+template <> struct PanelLds<float, true> {
+    float H[16][kHP];
+    int32_t step;
+    __device__ __forceinline__ void start() { if (threadIdx.x == 0) step = 0; }   // (a barrier follows)
+    template <int NW>
+    __device__ __forceinline__ bool run(float *G, int gp, int NP, int n, int k0, int w, int32_t *miss_sh) {
+        if constexpr (NW > 4) return panel_rows<NW>(G, gp, NP, n, k0, w, H, miss_sh);
+        else return panel_replay<NW>(G, gp, NP, n, k0, w, H, &step, miss_sh);
+    }
+};
+
 // Raw buffer access to one block's slot: a byte offset at or beyond the
 // descriptor's size (kOob) reads 0 and drops the store, so masked lanes need
 // no branch (descriptor word 3: raw, untyped access on CDNA).
@@ -860,7 +1005,7 @@ __device__ void ginv_pivot_body(T *__restrict__ M, T *__restrict__ S, int n, T *
 }
 
 // Wide-panel inverse with the pivot rows in registers: panels of H 16-column
-// halves in LDS (each half's Gauss-Jordan steps, panel_steps, then their
+// halves in LDS (each half's Gauss-Jordan steps, PanelLds::run, then their
 // transform on the other halves on MFMA), then every tile outside the panel
 // takes the rank-16H update.
 // Each wave owns whole tile columns; before updating any tile of a column it
@@ -876,9 +1021,9 @@ __device__ void ginv_pivot_body(T *__restrict__ M, T *__restrict__ S, int n, T *
 // update 347 -> 256, 205 of them products, with offsets that take one addition per
 // access); FP64, 40 blocks: 700 -> 501.
 template <typename T> struct GinvHalves { static constexpr int H = sizeof(T) == 4 ? 4 : 3; };
-template <typename T, int NR, int NTH, int UB, int H>
-__device__ bool ginv_body_wide_rx(T *__restrict__ M, T *__restrict__ S, int n, T *G, T (*Ws)[17],
-                                  T (*Ls)[17], int32_t *flag_sh) {
+template <typename T, int NR, int NTH, int UB, int H, bool REPLAY>
+__device__ bool ginv_body_wide_rx(T *__restrict__ M, T *__restrict__ S, int n, T *G, PanelLds<T, REPLAY> &pl,
+                                  int32_t *flag_sh) {
     typedef typename Mfma<T>::acc_t acc_t;
     constexpr int GP = 17, NWV = NTH / 64, PW = 16 * H;
     const int NT = (n + 15) / 16, NP = 16 * NT;
@@ -887,6 +1032,7 @@ __device__ bool ginv_body_wide_rx(T *__restrict__ M, T *__restrict__ S, int n, T
     const int nn = n * n;
     auto half = [&](int h) -> T * { return G + (size_t)h * NP * GP; };
     if (tid == 0) *flag_sh = 0;
+    pl.start();
     __syncthreads();
     // the first panel reads the block, the last one writes it, the others work in the
     // slot (M stays as it was until the last panel's pivots have passed their check)
@@ -918,7 +1064,7 @@ __device__ bool ginv_body_wide_rx(T *__restrict__ M, T *__restrict__ S, int n, T
         //    pivot-row operands every wave reads before any tile changes
         for (int h = 0; h < np; ++h) {
             const int kh = k0 + 16 * h, wh = width(h);
-            if (panel_steps<T, NWV>(half(h), GP, NP, n, kh, wh, Ws, Ls, flag_sh)) return false;
+            if (pl.template run<NWV>(half(h), GP, NP, n, kh, wh, flag_sh)) return false;
             if (np == 1) break;
             T b[H][4];
 #pragma unroll
@@ -1049,20 +1195,21 @@ __device__ bool ginv_body_wide_rx(T *__restrict__ M, T *__restrict__ S, int n, T
 constexpr int kInvThreads = 512;    // partial-pivoting inverse (k_fac_pivot): 8 waves per block
 constexpr int kWideThreads = 1024;   // wide-panel inverse: 16 waves per block
 
-template <typename T, int NR, int UB>
+template <typename T, int NR, int UB, bool REPLAY>
 __global__ void __launch_bounds__(kWideThreads) k_fac_ginv(T *__restrict__ D, int64_t ld, T *__restrict__ Wk, int64_t ldw,
                                                    const int32_t *__restrict__ rows, int n,
                                                    int32_t *__restrict__ redo) {
     extern __shared__ unsigned char smem_raw[];
     __shared__ int32_t flag_sh;
-    __shared__ T Ws[16][17], Ls[16][17];
+    __shared__ __attribute__((aligned(16))) unsigned char pl_raw[sizeof(PanelLds<T, REPLAY>)];
+    PanelLds<T, REPLAY> &pl = *reinterpret_cast<PanelLds<T, REPLAY> *>(pl_raw);
     const int blk = rows[blockIdx.x];
     T *M = D + (size_t)blk * ld;
     T *S = Wk + (size_t)blockIdx.x * ldw;
     // panels of GinvHalves<T>::H 16-column halves, pivot rows in registers (LDS: ginv_lds)
     constexpr int H = GinvHalves<T>::H;
     T *G = reinterpret_cast<T *>(smem_raw);                 // H * NP * 17
-    const bool ok = ginv_body_wide_rx<T, NR, kWideThreads, UB, H>(M, S, n, G, Ws, Ls, &flag_sh);
+    const bool ok = ginv_body_wide_rx<T, NR, kWideThreads, UB, H, REPLAY>(M, S, n, G, pl, &flag_sh);
     if (!ok && threadIdx.x == 0) redo[blk] = 1;    // left to k_fac_pivot; M untouched
 }
 
@@ -1075,7 +1222,7 @@ __global__ void __launch_bounds__(kWideThreads) k_fac_ginv(T *__restrict__ D, in
 // panels of 16:
 //   1. the panel's tiles go to LDS (G), and so do the other tiles of the
 //      panel's pivot rows k0..k0+15 (XP);
-//   2. panel_steps runs the checked-diagonal Gauss-Jordan on the n x 16 panel,
+//   2. PanelLds::run takes the checked-diagonal Gauss-Jordan steps on the n x 16 panel,
 //      which then holds C = [W on the pivot rows P, -A(r,P) W elsewhere], W
 //      the inverse of the panel's pivot block;
 //   3. every other column is updated at once, X += (C - E_P) X(P,:), one
@@ -1143,7 +1290,7 @@ __device__ __forceinline__ void store48(T (&X)[kRowN][P], const Fetched48<S> &f,
     }
 }
 
-template <typename T, int NT, typename SB = void>
+template <typename T, int NT, typename SB = void, bool REPLAY = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 k_fac_binv(T *__restrict__ D, int64_t ld, const int32_t *__restrict__ rows, int n, int32_t *__restrict__ err,
            RowIn<T, SB> in) {
@@ -1159,7 +1306,8 @@ k_fac_binv(T *__restrict__ D, int64_t ld, const int32_t *__restrict__ rows, int 
     constexpr int XPP = NP + 1;                  // LDS pitch of the pivot rows
     __shared__ T G[NP * GP];                     // panel in, C - E_P out
     __shared__ T XP[16 * XPP];                   // pivot rows of the other columns
-    __shared__ T Ws[16][17], Ls[16][17];         // of the panel's pivot block (panel_steps)
+    __shared__ __attribute__((aligned(16))) unsigned char pl_raw[sizeof(PanelLds<T, REPLAY>)];   // of the panel's steps
+    PanelLds<T, REPLAY> &pl = *reinterpret_cast<PanelLds<T, REPLAY> *>(pl_raw);
     __shared__ int32_t miss_sh;
     typedef typename Mfma<T>::acc_t acc_t;
     const int blk = rows[blockIdx.x];
@@ -1276,6 +1424,7 @@ k_fac_binv(T *__restrict__ D, int64_t ld, const int32_t *__restrict__ rows, int 
     }
     for (int e = tid; e < 16 * XPP; e += 256) XP[e] = T(0);
     if (tid == 0) miss_sh = 0;
+    pl.start();
     // B operand of the identity: I[4kk + lane/16][lane%16]
     T ident[4];
 #pragma unroll
@@ -1333,7 +1482,7 @@ k_fac_binv(T *__restrict__ D, int64_t ld, const int32_t *__restrict__ rows, int 
             for (int kk = 0; kk < 4; ++kk) bx[x][kk] = XP[(4 * kk + (lane >> 4)) * XPP + 16 * etj + (lane & 15)];
         }
         // 2. panel Gauss-Jordan (checked diagonal pivots)
-        if (panel_steps<T, 4>(G, GP, NP, n, k0, w, Ws, Ls, &miss_sh)) break;
+        if (pl.template run<4>(G, GP, NP, n, k0, w, &miss_sh)) break;
         // 3. X += (C - E_P) X(P,:) on MFMA; the panel's tiles take C
         auto ldA = [&](int ti, int kk) -> T { return G[(16 * ti + (lane & 15)) * GP + 4 * kk + (lane >> 4)]; };
         auto panel_tile = [&](const T (&av)[4], int ti) -> acc_t {
@@ -1514,6 +1663,9 @@ __global__ void k_f32_to_bf16(const float *__restrict__ src, cdg_bf16 *__restric
         dst[k] = to_bf16(src[k]);
 }
 
+// BF16-stored factors are computed in FP32 and take the REPLAY panels.
+template <typename T> constexpr bool kReplays = sizeof(T) == 4;
+
 template <typename T, int NR>
 int launch_ginv(cdg_ctx *ctx, cdg_prec *M, T *D, int64_t ld, const int32_t *rows, int nrows_lvl, int n,
                 int32_t *err) {
@@ -1528,20 +1680,23 @@ int launch_ginv(cdg_ctx *ctx, cdg_prec *M, T *D, int64_t ld, const int32_t *rows
         const int v = e ? std::atoi(e) : 2;
         return v <= 2 ? 2 : v <= 4 ? 4 : 8;
     }();
-    const void *fn = ub == 2 ? reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 2>)
-                   : ub == 4 ? reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 4>)
-                             : reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 8>);
+    static const void *const fns[2][3] = {
+        {reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 2, false>), reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 4, false>),
+         reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 8, false>)},
+        {reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 2, kReplays<T>>), reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 4, kReplays<T>>),
+         reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 8, kReplays<T>>)}};
+    const void *fn = fns[M->precision == CDG_BF16][ub == 2 ? 0 : ub == 4 ? 1 : 2];
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
     std::call_once(once, [] {
         const int most = (int)ginv_lds<T, NR>(std::min(64 * NR, 320));
-        const void *fns[] = {reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 2>),
-                             reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 4>),
-                             reinterpret_cast<const void *>(&k_fac_ginv<T, NR, 8>),
-                             reinterpret_cast<const void *>(&k_fac_pivot<T, NR>)};
-        for (const void *f : fns)
+        auto set = [&](const void *f) {
             if (attr_err == hipSuccess)
                 attr_err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+        };
+        for (auto &r : fns)
+            for (const void *f : r) set(f);
+        set(reinterpret_cast<const void *>(&k_fac_pivot<T, NR>));
     });
     if (attr_err != hipSuccess)
         return cdg_fail(ctx, CDG_ERR_HIP, "hipFuncSetAttribute (block inverse LDS): %s", hipGetErrorString(attr_err));
@@ -1588,8 +1743,13 @@ int launch_inv(cdg_ctx *ctx, cdg_prec *M, T *D, int64_t ld, const int32_t *rows,
     dim3 grid(nrows_lvl), block(256);
     if (mode == 1 && n <= 144) {
         const RowIn<T, void> in{static_cast<T *>(M->inv_w), M->d_redo};
-        if (n <= 96) hipLaunchKernelGGL((k_fac_binv<T, 6>), grid, block, 0, ctx->stream, D, ld, rows, n, err, in);
-        else hipLaunchKernelGGL((k_fac_binv<T, 9>), grid, block, 0, ctx->stream, D, ld, rows, n, err, in);
+        auto go = [&](auto rp) {
+            constexpr bool RP = decltype(rp)::value;
+            if (n <= 96) hipLaunchKernelGGL((k_fac_binv<T, 6, void, RP>), grid, block, 0, ctx->stream, D, ld, rows, n, err, in);
+            else hipLaunchKernelGGL((k_fac_binv<T, 9, void, RP>), grid, block, 0, ctx->stream, D, ld, rows, n, err, in);
+        };
+        if (M->precision == CDG_BF16) go(std::integral_constant<bool, kReplays<T>>{});
+        else go(std::false_type{});
         CDG_HIP_TRY(hipGetLastError());
         if (n <= 96 || kPivotsHere<T, 9>) return CDG_OK;
         const size_t lds = ginv_lds<T, 3>(n);
@@ -1675,7 +1835,9 @@ int row_level(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, T *L, T *D, const flo
         in.lo_blk = M->d_lo_blk;
         in.lo_col = M->d_lo_col;
         in.diag = M->d_diag;
-        hipLaunchKernelGGL((k_fac_binv<T, kRowN / 16, SB>), dim3(r1 - r0), dim3(256), 0, ctx->stream, D, M->ld, rows, M->n,
+        // (FP32 from A's FP64 blocks: BF16 storage)
+        constexpr bool RP = sizeof(T) == 4 && std::is_same<SB, double>::value;
+        hipLaunchKernelGGL((k_fac_binv<T, kRowN / 16, SB, RP>), dim3(r1 - r0), dim3(256), 0, ctx->stream, D, M->ld, rows, M->n,
                            M->d_err, in);
     };
     bool done = false;
