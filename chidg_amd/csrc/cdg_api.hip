@@ -1415,6 +1415,16 @@ int solve_lanes(cdg_ctx *ctx, const cdg_mat *A, cdg_prec *M, int k, const double
         t_factor = secs(tf, clk::now());
     }
     const int64_t len = (int64_t)A->nrows * A->n;
+    if (len == 0) {   // no rows: x = (), nothing to launch (the step's kernels need a value)
+        if (prm->nkrylov < 1) return cdg_fail(ctx, CDG_ERR_ARG, "nkrylov must be >= 1");
+        for (int r = 0; r < k; ++r) {
+            std::memset(&st[r], 0, sizeof(st[r]));
+            st[r].factored = factored;
+            st[r].t_factor = t_factor;
+            st[r].t_total = secs(t_start, clk::now());
+        }
+        return CDG_OK;
+    }
     VecArg bi, xo;
     e = stage_in(ctx, 0, b, len * k, bi);
     if (!e) e = stage_in(ctx, 1, x, len * k, xo);

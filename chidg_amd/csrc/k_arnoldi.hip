@@ -480,7 +480,7 @@ __global__ void k_stamp(uint64_t *p) { *p = wall_clock64(); }
 
 }  // namespace
 
-// Workspace of one FGMRES level: nl lanes, up to m steps, vectors of len values.
+// Workspace of one FGMRES level: nl lanes, up to m steps, vectors of len >= 1 values.
 int arn_alloc(cdg_ctx *ctx, Arnoldi &A, int nl, int m, int64_t len, bool mgs) {
     A.nl = nl;
     A.m = m;
