@@ -371,12 +371,6 @@ extern "C" int cdg_ctx_create(int32_t device, cdg_ctx **out) {
     }
     if (const char *sp = std::getenv("CDG_SPIN")) ctx->spin = std::atoi(sp) != 0;
     if (ctx_ensure_small(ctx, 4096) || ctx_ensure_part(ctx, 1 << 16)) { cdg_ctx_destroy(ctx); return CDG_ERR_OOM; }
-    if (hipHostMalloc((void **)&ctx->h_sweep_err, 64) != hipSuccess) {
-        ctx->h_sweep_err = nullptr;
-        cdg_ctx_destroy(ctx);
-        return CDG_ERR_OOM;
-    }
-    *ctx->h_sweep_err = 0;
     *out = ctx;
     return CDG_OK;
 }
@@ -395,7 +389,7 @@ extern "C" int cdg_ctx_destroy(cdg_ctx *ctx) {
     if (ctx->done_ev) (void)hipEventDestroy(ctx->done_ev);
     if (ctx->order_ev) (void)hipEventDestroy(ctx->order_ev);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-    if (ctx->h_sweep_err) (void)hipHostFree(ctx->h_sweep_err);
+    for (uint32_t *p : ctx->word_pages) (void)hipHostFree(p);
     if (ctx->h_arn) (void)hipHostFree(ctx->h_arn);
     delete ctx;
     return CDG_OK;
@@ -631,6 +625,7 @@ extern "C" int cdg_prec_destroy(cdg_ctx *ctx, cdg_prec *M) {
     if (ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         for (DevMem &m : M->owned) dev_free(ctx, m.p, m.bytes);
+        if (M->h_err) ctx->word_free.push_back(M->h_err);
     }
     sweep_free(M);
     delete M;
@@ -782,6 +777,21 @@ extern "C" int cdg_prec_create(cdg_ctx *ctx, const cdg_mat *A, int32_t type, int
     M->part_cap = part_doubles;
     if (!e && M->apply_mode == CDG_APPLY_DATAFLOW) e = df_setup(ctx, M);
     if (!e && M->apply_mode == CDG_APPLY_FOLDED) e = alloc(&M->W, es * (size_t)M->nup * M->ld);
+    if (!e && ctx->word_free.empty()) {
+        uint32_t *page = nullptr;
+        constexpr size_t kWords = 64, kPitch = 16;   // a word per cache line
+        if (hipHostMalloc((void **)&page, sizeof(uint32_t) * kWords * kPitch) == hipSuccess) {
+            ctx->word_pages.push_back(page);
+            for (size_t i = 0; i < kWords; ++i) ctx->word_free.push_back(page + kPitch * i);
+        } else {
+            e = cdg_fail(ctx, CDG_ERR_OOM, "pinned error words");
+        }
+    }
+    if (!e) {
+        M->h_err = ctx->word_free.back();
+        ctx->word_free.pop_back();
+        *M->h_err = 0;
+    }
     if (const char *f = std::getenv("CDG_FOLD_AFTER")) M->fold_after = std::max(0, std::atoi(f));
     if (!e) {   // the single-vector sweep's plans and W, so that an apply never allocates
         SweepPlan *p = nullptr;
@@ -1016,12 +1026,17 @@ extern "C" int cdg_mat_launch_shape(const cdg_mat *A, int32_t *out) {
     return CDG_OK;
 }
 
+// An abandoned wait left NaN in z and raised its preconditioner's word (call when the stream is idle).
+int sweep_check(cdg_ctx *ctx, cdg_prec *M) {
+    if (M->h_err && __atomic_exchange_n(M->h_err, 0u, __ATOMIC_ACQ_REL) != 0)
+        return cdg_fail(ctx, CDG_ERR_HIP, "ILU(0) sweep gave up waiting for a dependency");
+    return CDG_OK;
+}
+
 // A dataflow sweep that gave up waiting leaves its counters unusable: report
 // it and reset them (called from the synchronizing entry points).
 static int df_check(cdg_ctx *ctx, cdg_prec *M) {
-    // the sweep: an abandoned wait left NaN in z and raised the context's flag
-    if (__atomic_exchange_n(ctx->h_sweep_err, 0u, __ATOMIC_ACQ_REL) != 0)
-        return cdg_fail(ctx, CDG_ERR_HIP, "ILU(0) sweep gave up waiting for a dependency");
+    if (int e = sweep_check(ctx, M)) return e;
     if (M->apply_mode != CDG_APPLY_DATAFLOW || !M->d_dferr) return CDG_OK;
     int32_t err = 0;
     CDG_HIP_TRY(hipMemcpyAsync(&err, M->d_dferr, sizeof(err), hipMemcpyDeviceToHost, ctx->stream));
@@ -1472,8 +1487,7 @@ int solve_lanes(cdg_ctx *ctx, const cdg_mat *A, cdg_prec *M, int k, const double
     for (int r = 0; r < k && !e; ++r)
         if (!std::isfinite(st[r].residual_norm)) e = cdg_fail(ctx, CDG_ERR_NAN, "non-finite final residual");
     for (Level &l : lvs) level_free(ctx, l);
-    // a sweep that gave up left NaN behind
-    if (e != CDG_OK || *ctx->h_sweep_err) {
+    if (e == CDG_ERR_NAN) {   // a sweep that gave up left NaN behind
         const int e2 = df_check(ctx, M);
         if (e2) return e2;
     }

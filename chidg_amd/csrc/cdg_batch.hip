@@ -678,9 +678,8 @@ extern "C" int cdg_batch_destroy(cdg_ctx *ctx, cdg_batch *bt) {
     return CDG_OK;
 }
 
-extern "C" int cdg_batch_solve(cdg_ctx *ctx, cdg_batch *bt, const double *const *b, double *const *x,
-                               const cdg_fgmres_params *prm, cdg_fgmres_stats *stats) {
-    if (!ctx || !bt || !b || !x || !prm) return CDG_ERR_ARG;
+static int batch_run(cdg_ctx *ctx, cdg_batch *bt, const double *const *b, double *const *x,
+                     const cdg_fgmres_params *prm, cdg_fgmres_stats *stats) {
     if (prm->nkrylov != bt->m) return cdg_fail(ctx, CDG_ERR_ARG, "batch: nkrylov %d, created with %d", prm->nkrylov, bt->m);
     if (prm->inner_fgmres || prm->orthogonalization != CDG_CGS)
         return cdg_fail(ctx, CDG_ERR_UNSUPPORTED, "batch: CGS without inner FGMRES only");
@@ -902,6 +901,17 @@ extern "C" int cdg_batch_solve(cdg_ctx *ctx, cdg_batch *bt, const double *const 
             o.t_total = t;
         }
     }
+    return e;
+}
+
+extern "C" int cdg_batch_solve(cdg_ctx *ctx, cdg_batch *bt, const double *const *b, double *const *x,
+                               const cdg_fgmres_params *prm, cdg_fgmres_stats *stats) {
+    if (!ctx || !bt || !b || !x || !prm) return CDG_ERR_ARG;
+    int e = batch_run(ctx, bt, b, x, prm, stats);
+    if (e) (void)hipStreamSynchronize(ctx->stream);
+    // a sweep that gave up waiting is the cause of what was found (the words of every group are cleared)
+    for (BatchGroup &g : bt->groups)
+        if (const int e2 = sweep_check(ctx, g.M)) e = e2;
     return e;
 }
 

@@ -58,7 +58,9 @@ struct cdg_ctx {
     int arn_cap = 0;
     uint64_t *hook_stamp = nullptr;
     const int *hook_nact = nullptr;
-    uint32_t *h_sweep_err = nullptr;   // pinned: raised by an ILU(0) sweep that gave up waiting
+    // pinned words, one per preconditioner, that a sweep which gave up waiting raises: the pages, and
+    // those of their words that no preconditioner holds
+    std::vector<uint32_t *> word_pages, word_free;
 };
 
 // Waits until the context's stream has finished its work: polls a completion
@@ -181,6 +183,7 @@ struct cdg_prec {
     int32_t fold_ok = 0, fold_after = 12, napply = 0, prev_napply = 0;
     int32_t w_asked = 0;               // W of this factor was asked for by name or for several vectors
     int32_t w_keep = 0;                // a captured launch reads W: every update forms it anew
+    uint32_t *h_err = nullptr;         // pinned: raised by one of its sweeps that gave up waiting
     int32_t noalloc_ok = 0;            // CDG_SCHEDULE_ROWSLICE or _STREAM was set (cdg_prec_apply_noalloc)
     uint64_t stamp = 0;
     int32_t factored = 0;
@@ -241,6 +244,7 @@ enum { CDG_APPLY_LEVELS = 0, CDG_APPLY_DATAFLOW = 1, CDG_APPLY_FOLDED = 2, CDG_A
 bool sweep_shape(int n, int precision, int maxdep, int width, int cus, SweepShape *out);
 int sweep_plan(cdg_ctx *ctx, cdg_prec *M, int K, int lo, int hi, bool fold, SweepPlan **out);
 int sweep_fold(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A);
+int sweep_check(cdg_ctx *ctx, cdg_prec *M);   // an error if a sweep of M has given up since the last look
 void sweep_free(cdg_prec *M);
 int launch_ilu_sweep(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t stride, int k,
                      bool fold, const int32_t *row_k = nullptr, int lo = 0, int hi = -1);
