@@ -248,6 +248,8 @@ int sweep_check(cdg_ctx *ctx, cdg_prec *M);   // an error if a sweep of M has gi
 void sweep_free(cdg_prec *M);
 int launch_ilu_sweep(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t stride, int k,
                      bool fold, const int32_t *row_k = nullptr, int lo = 0, int hi = -1);
+int launch_diag(cdg_ctx *ctx, const cdg_prec *M, const double *v, double *z, int64_t stride, int k, const int32_t *row_k,
+                int lo, int hi);
 int launch_fold_left(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A);
 int launch_mv_multi(cdg_ctx *ctx, const cdg_mat *A, const double *X, double *Y, int64_t stride, int k,
                     const int32_t *row_k = nullptr, int row_lo = 0, int row_hi = -1);

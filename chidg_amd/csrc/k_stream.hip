@@ -418,6 +418,53 @@ __global__ void k_sum_parts(const PT *__restrict__ part, int S, int n, int64_t l
     }
 }
 
+__device__ __forceinline__ double widen(double x) { return x; }
+__device__ __forceinline__ double widen(float x) { return x; }
+__device__ __forceinline__ double widen(cdg_bf16 x) { return __uint_as_float(static_cast<uint32_t>(x) << 16); }
+
+// The ILU(0) apply where no row has lower or upper blocks (block Jacobi): z_i = Dinv_i v_i for up
+// to K right-hand sides, FP64 sums over the stored values.  Thread (i, r) sums row r of block i over its
+// columns, so a wavefront reads whole columns and nothing is reduced; a workgroup takes as many
+// rows i as fit 256 threads.  What bounds it: the reads of Dinv.  The sweep spends two tasks of
+// a hop's length on such a row: 30^3 P1 FP64 717 us, here 69 (level launches 197); 16^3 P2 FP64 428,
+// here 125 (273), FP32 199 and 56; eight vectors 1588 and 158.
+template <typename S, int K>
+__global__ void __launch_bounds__(512) k_diag(const S *__restrict__ D, int64_t ld, const double *v, double *z,
+                                              int64_t stride, int n, int per, int k,
+                                              const int32_t *__restrict__ row_k, int r0, int lo, int hi,
+                                              const int *__restrict__ nact, uint64_t *__restrict__ stamp) {
+    if (nact && *nact == 0) return;   // a step queued after every right-hand side stopped
+    if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+    extern __shared__ double smem[];  // per * n values, K right-hand sides each
+    const int i = threadIdx.x / n, r = threadIdx.x - i * n, row = lo + (int)blockIdx.x * per + i;
+    const bool on = i < per && row < hi;
+    const int kr = on ? min(row_k ? row_k[row] - r0 : k, K) : 0;
+    if (on)
+#pragma unroll
+        for (int q = 0; q < K; ++q) smem[threadIdx.x * K + q] = q < kr ? v[q * stride + (int64_t)row * n + r] : 0.0;
+    __syncthreads();
+    if (kr <= 0) return;
+    const S *const col = D + (size_t)row * ld + r;
+    const double *const x = smem + (size_t)i * n * K;
+    double acc[K];
+#pragma unroll
+    for (int q = 0; q < K; ++q) acc[q] = 0.0;
+    constexpr int U = 16;             // columns in flight
+    for (int c0 = 0; c0 < n; c0 += U) {
+        S d[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) d[u] = col[(size_t)min(c0 + u, n - 1) * n];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (c0 + u < n)
+#pragma unroll
+                for (int q = 0; q < K; ++q) acc[q] += widen(d[u]) * x[(c0 + u) * K + q];
+    }
+#pragma unroll
+    for (int q = 0; q < K; ++q)
+        if (q < kr) z[q * stride + (int64_t)row * n + r] = acc[q];
+}
+
 // Identity preconditioner / widening copy: dst[k] = (double) src[k]
 template <typename S>
 __global__ void k_widen(const S *__restrict__ src, double *__restrict__ dst, int64_t count) {
@@ -627,4 +674,41 @@ int launch_widen(cdg_ctx *ctx, const void *src, int precision, double *dst, int6
         hipLaunchKernelGGL(k_widen<cdg_bf16>, grid, block, 0, ctx->stream, static_cast<const cdg_bf16 *>(src), dst, count);
     CDG_HIP_TRY(hipGetLastError());
     return CDG_OK;
+}
+
+namespace {
+template <typename S, int K>
+void diag_k(cdg_ctx *ctx, const cdg_prec *M, const double *v, double *z, int64_t stride, int k, const int32_t *row_k,
+            int r0, int lo, int hi) {
+    const int n = M->n, per = std::max(1, 256 / n), rows = hi - lo;
+    const dim3 grid((rows + per - 1) / per), blk((per * n + 63) / 64 * 64);
+    hipLaunchKernelGGL((k_diag<S, K>), grid, blk, sizeof(double) * blk.x * K, ctx->stream, static_cast<const S *>(M->Dinv),
+                       M->ld, v, z, stride, n, per, k, row_k, r0, lo, hi, ctx->hook_nact,
+                       r0 == 0 ? ctx->hook_stamp : nullptr);
+}
+template <typename S>
+int diag_s(cdg_ctx *ctx, const cdg_prec *M, const double *v, double *z, int64_t stride, int k, const int32_t *row_k,
+           int lo, int hi) {
+    for (int r0 = 0; r0 < k; r0 += 8) {
+        const int kk = std::min(8, k - r0);
+        const double *vr = v + (size_t)r0 * stride;
+        double *zr = z + (size_t)r0 * stride;
+        if (kk == 1) diag_k<S, 1>(ctx, M, vr, zr, stride, kk, row_k, r0, lo, hi);
+        else if (kk == 2) diag_k<S, 2>(ctx, M, vr, zr, stride, kk, row_k, r0, lo, hi);
+        else if (kk <= 4) diag_k<S, 4>(ctx, M, vr, zr, stride, kk, row_k, r0, lo, hi);
+        else diag_k<S, 8>(ctx, M, vr, zr, stride, kk, row_k, r0, lo, hi);
+        CDG_HIP_TRY(hipGetLastError());
+    }
+    return CDG_OK;
+}
+}  // namespace
+
+// z_r = Dinv v_r for r < k, rows [lo, hi): the whole apply where M has no lower and upper blocks.
+// Each right-hand side gets the bits it gets alone.
+int launch_diag(cdg_ctx *ctx, const cdg_prec *M, const double *v, double *z, int64_t stride, int k, const int32_t *row_k,
+                int lo, int hi) {
+    if (hi <= lo) return CDG_OK;
+    return M->precision == CDG_FP64 ? diag_s<double>(ctx, M, v, z, stride, k, row_k, lo, hi)
+         : M->precision == CDG_FP32 ? diag_s<float>(ctx, M, v, z, stride, k, row_k, lo, hi)
+                                    : diag_s<cdg_bf16>(ctx, M, v, z, stride, k, row_k, lo, hi);
 }
