@@ -241,7 +241,7 @@ int df_reset(cdg_ctx *ctx, cdg_prec *M);
 enum { CDG_APPLY_LEVELS = 0, CDG_APPLY_DATAFLOW = 1, CDG_APPLY_FOLDED = 2, CDG_APPLY_AUTO = 3, CDG_APPLY_STREAM = 4,
        CDG_APPLY_ROWSLICE = 5 };
 // the sweep (k_sweep.hip)
-bool sweep_shape(int n, int precision, int maxdep, int width, int cus, SweepShape *out);
+bool sweep_shape(int n, int precision, int maxdep, int width, int mean, int cus, SweepShape *out);
 int sweep_plan(cdg_ctx *ctx, cdg_prec *M, int K, int lo, int hi, bool fold, SweepPlan **out);
 int sweep_fold(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A);
 int sweep_check(cdg_ctx *ctx, cdg_prec *M);   // an error if a sweep of M has given up since the last look

@@ -142,12 +142,12 @@ static int64_t factor_extra_bytes(int64_t nrows, int64_t nlo, int64_t n, int pre
     if (n > 192) f += 8 * nrows * ld;                            // inverse working slots (bound)
     f += 3 * 8 * nrows * 8 * n;                                  // apply partial sums (<= 8 slices)
     SweepShape sh;                                               // the sweep's exchange words and task records
-    if (sweep_shape((int)n, precision, precision == CDG_BF16 ? 4 : 3, 1, 256, &sh))
+    if (sweep_shape((int)n, precision, precision == CDG_BF16 ? 4 : 3, 1, 1, 256, &sh))
         for (int64_t k = 1; k <= 8; k *= 8)                      // one vector, and up to eight together
             f += 8 * 6 * sh.C * k * len + 64 * (3 * sh.C + 1) * nrows;
     if (precision == CDG_BF16) {                                 // the folded form: W, one more single-vector plan
         f += es * nlo * ld;
-        if (sweep_shape((int)n, precision, 4, 1, 256, &sh)) f += 8 * 6 * sh.C * len + 64 * (2 * sh.C + 1) * nrows;
+        if (sweep_shape((int)n, precision, 4, 1, 1, 256, &sh)) f += 8 * 6 * sh.C * len + 64 * (2 * sh.C + 1) * nrows;
     }
     return f;
 }
