@@ -1375,7 +1375,7 @@ int fgmres_lanes(Solver &S, std::vector<Level> &lvs, int depth, int k, const dou
                 // zr = v_j - A z_j ; inner solve ; z_j += dz   (:179-183)
                 ctx->hook_nact = nullptr;
                 ctx->hook_stamp = nullptr;
-                std::vector<int> nr;
+                std::vector<int> nr(1, 0);                 // (its restarts are not reported)
                 e = launch_mv(ctx, S.A, zj, lv.zr);
                 if (!e) e = kv_sub(ctx, len, vj, lv.zr, lv.zr);
                 if (!e) e = fgmres_lanes(S, lvs, depth + 1, 1, lv.zr, lv.dz, inner->inner_nkrylov, inner->inner_tol,
