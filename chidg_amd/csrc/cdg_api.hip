@@ -1459,6 +1459,7 @@ int solve_lanes(cdg_ctx *ctx, const cdg_mat *A, cdg_prec *M, int k, const double
     if (!e) {
         lv.arn.a.b = bi.dev;
         lv.arn.a.ax = lv.r0;
+        lv.arn.a.inner_st = lvs[1].arn.a.st;
         e = arn_launch(ctx, lv.arn, ARN_NORM, 0);
     }
     if (!e) e = arn_wait(ctx, ctx->h_arn, k, lv.arn.a.seq);

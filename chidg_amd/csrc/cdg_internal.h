@@ -192,7 +192,7 @@ struct cdg_prec {
 
 // ---- the vector part of FGMRES steps (k_arnoldi.hip) --------------------------
 enum { ARN_CGS = 0, ARN_MGS = 1, ARN_START = 2, ARN_NORM = 3 };
-enum { ARN_ACTIVE, ARN_DONE, ARN_NVECS, ARN_NITER, ARN_CONV, ARN_NREORTH, ARN_SECOND, ARN_RUN, ARN_NST = 32 };   // int state of a lane (a line)
+enum { ARN_ACTIVE, ARN_DONE, ARN_NVECS, ARN_NITER, ARN_CONV, ARN_NREORTH, ARN_SECOND, ARN_RUN, ARN_NREALL, ARN_NST = 32 };   // int state of a lane (a line); NREALL: second passes of all solves on this workspace
 enum { ARN_R0INIT, ARN_RES, ARN_TP, ARN_TM, ARN_TO, ARN_TN, ARN_NSC = 16 };                 // doubles of a lane
 // What launches report per lane, in pinned memory: after each step one word, the
 // launch's number, the lane's steps in this cycle and ARN_W_* bits; the rest with the word of an
@@ -213,6 +213,7 @@ struct ArnArgs {
     double *part, *sums;          // [lane][value][slice], [lane][value]
     uint64_t *stamp;
     int *nact;                    // lanes still running
+    const int *inner_st;          // NORM: null, or the state of the nested solver's lane
     ArnRes *hres;
     uint32_t seq;
     double tol, rtol;

@@ -356,7 +356,10 @@ __global__ void __launch_bounds__(256) k_arn_finish(ArnArgs a) {
             res = fabs(-s1 * pj);
             const int it = ++st[ARN_NITER];
             st[ARN_NVECS] = jj;
-            if (second) ++st[ARN_NREORTH];
+            if (second) {
+                ++st[ARN_NREORTH];
+                ++st[ARN_NREALL];
+            }
             const bool ca = res < a.tol, cr = (res / sc[ARN_R0INIT]) < a.rtol, cn = it >= a.nmax && a.nmax > 0;
             if (!isfinite(res)) err = 1;
             else if (ca || cr || cn) conv = 1;
@@ -395,7 +398,7 @@ __global__ void __launch_bounds__(256) k_arn_finish(ArnArgs a) {
             put(&o->t[2], sc[ARN_TO]);
             put(&o->t[3], sc[ARN_TN]);
             put(&o->niter, st[ARN_NITER]);
-            put(&o->nreorth, st[ARN_NREORTH]);
+            put(&o->nreorth, st[ARN_NREORTH] + (a.inner_st ? a.inner_st[ARN_NREALL] : 0));
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_s_waitcnt(0);              // before the word that announces it
         } else {

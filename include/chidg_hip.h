@@ -87,7 +87,8 @@ typedef struct {
     int32_t niter;
     double  residual_norm;           /* ||b - A x|| after the solve           */
     int32_t nrestart;
-    int32_t nreorth;                 /* re-orthogonalized Arnoldi steps        */
+    int32_t nreorth;                 /* re-orthogonalized Arnoldi steps, those of
+                                        the nested solver included             */
     int32_t factored;                /* 1 if the preconditioner was updated    */
     double  t_total;
     double  t_factor;
