@@ -1521,7 +1521,14 @@ extern "C" int cdg_fgmres_solve_multi(cdg_ctx *ctx, const cdg_mat *A, cdg_prec *
         return CDG_OK;
     }
     std::vector<cdg_fgmres_stats> local(k);
-    const int e = solve_lanes(ctx, A, M, k, b, x, prm, local.data());
+    // the step's kernels have a grid row per vector: 65535 at most
+    constexpr int32_t kMost = 32768;
+    int e = CDG_OK;
+    for (int32_t r = 0; r < k && !e; r += kMost) {
+        cdg_fgmres_params p1 = *prm;
+        if (r > 0) p1.update_preconditioner = 0;
+        e = solve_lanes(ctx, A, M, std::min(kMost, k - r), b + (size_t)r * len, x + (size_t)r * len, &p1, local.data() + r);
+    }
     if (st) std::memcpy(st, local.data(), sizeof(cdg_fgmres_stats) * k);
     return e;
 }
