@@ -580,11 +580,30 @@ extern "C" int cdg_mv_async(cdg_ctx *ctx, const cdg_mat *A, const double *x, dou
 // ---------------------------------------------------------------------------
 // preconditioner
 // ---------------------------------------------------------------------------
+// The partial sums' storage of the column-slice schedules (FOLDED, DATAFLOW and the level
+// launches), at least 3 part_len doubles; the sweep has none.  (+2: a launch whose
+// rows have no entries issues its 16-byte block prefetch from the start of a partial
+// array, unused.)
+static int prec_part_fit(cdg_ctx *ctx, cdg_prec *M) {
+    const int64_t need = 3 * M->part_len + 2;
+    if (need <= M->part_cap) return CDG_OK;
+    double *np = nullptr;
+    const size_t bytes = sizeof(double) * (size_t)need;
+    int e = dev_alloc(ctx, (void **)&np, bytes);
+    if (e) return e;
+    if (!M->d_part) M->owned.push_back({np, bytes});
+    for (DevMem &m : M->owned)
+        if (M->d_part && m.p == M->d_part) { dev_free(ctx, m.p, m.bytes); m.p = np; m.bytes = bytes; }
+    M->d_part = np;
+    M->part_cap = need;
+    return CDG_OK;
+}
+
 // Task list, counters and partial storage of the dataflow sweep (once per
 // preconditioner).  Tickets: forward levels ascending; per backward level its
 // BA tasks then its BB tasks, so every input of a task has a smaller ticket.
 static int df_setup(cdg_ctx *ctx, cdg_prec *M) {
-    if (M->d_tasks) return CDG_OK;
+    if (M->d_tasks) return prec_part_fit(ctx, M);
     int e = df_configure(ctx, M);
     if (e) return e;
     const int S = M->df_S;
@@ -599,16 +618,9 @@ static int df_setup(cdg_ctx *ctx, cdg_prec *M) {
                 for (int sl = 0; sl < S; ++sl) tasks.push_back(((M->h_blev_rows[k] * S + sl) << 2) | stg);
     M->df_ntasks = (int32_t)tasks.size();
     const int64_t need = 3 * (int64_t)M->nrows * S * M->n;
-    if (need > 3 * M->part_len) {      // partial storage shared with the level schedule
-        double *np = nullptr;
-        e = dev_alloc(ctx, (void **)&np, sizeof(double) * (size_t)(need + 2));   // +2 as at init
-        if (e) return e;
-        for (DevMem &m : M->owned)
-            if (m.p == M->d_part) { dev_free(ctx, m.p, m.bytes); m.p = np; m.bytes = sizeof(double) * (size_t)(need + 2); }
-        M->d_part = np;
-        M->part_len = need / 3;
-        M->part_cap = need + 2;
-    }
+    M->part_len = std::max(M->part_len, need / 3);   // partial storage shared with the level schedule
+    e = prec_part_fit(ctx, M);
+    if (e) return e;
     e = upload_array(ctx, &M->d_tasks, tasks, &M->owned);
     if (!e) e = upload_array(ctx, &M->d_cnt, std::vector<int32_t>((size_t)3 * M->nrows, 0), &M->owned);
     if (!e) e = upload_array(ctx, &M->d_dferr, std::vector<int32_t>(1, 0), &M->owned);
@@ -770,11 +782,6 @@ extern "C" int cdg_prec_create(cdg_ctx *ctx, const cdg_mat *A, int32_t type, int
     M->h_up_col = S->up_col;
     M->h_up_idx = up_idx;
     M->h_blev_rows = border;
-    // (+2: a sweep launch whose rows have no entries issues its 16-byte
-    // block prefetch from the start of a partial array, unused)
-    const int64_t part_doubles = 3 * M->part_len + 2;
-    if (!e) e = alloc((void **)&M->d_part, sizeof(double) * (size_t)part_doubles);
-    M->part_cap = part_doubles;
     if (!e && M->apply_mode == CDG_APPLY_DATAFLOW) e = df_setup(ctx, M);
     if (!e && M->apply_mode == CDG_APPLY_FOLDED) e = alloc(&M->W, es * (size_t)M->nup * M->ld);
     if (!e && ctx->word_free.empty()) {
@@ -798,6 +805,7 @@ extern "C" int cdg_prec_create(cdg_ctx *ctx, const cdg_mat *A, int32_t type, int
         int ep = sweep_plan(ctx, M, 1, 0, M->nrows, false, &p);
         if (ep == CDG_ERR_UNSUPPORTED) M->sweep_ok = 0;
         else e = ep;
+        if (!e && (!M->sweep_ok || M->apply_mode == CDG_APPLY_FOLDED)) e = prec_part_fit(ctx, M);
         if (!e && M->sweep_ok && precision == CDG_BF16 && M->nup > 0 && M->maxdep <= 6) {
             ep = sweep_plan(ctx, M, 1, 0, M->nrows, true, &p);
             if (!ep) {
@@ -848,6 +856,8 @@ extern "C" int cdg_prec_set_schedule(cdg_ctx *ctx, cdg_prec *M, int32_t schedule
             if (e) return e;
             M->owned.push_back({M->W, bytes});
         }
+        int e = prec_part_fit(ctx, M);
+        if (e) return e;
     }
     M->apply_mode = schedule == CDG_SCHEDULE_DATAFLOW ? CDG_APPLY_DATAFLOW
                     : schedule == CDG_SCHEDULE_FOLDED ? CDG_APPLY_FOLDED
@@ -855,6 +865,14 @@ extern "C" int cdg_prec_set_schedule(cdg_ctx *ctx, cdg_prec *M, int32_t schedule
                     : schedule == CDG_SCHEDULE_ROWSLICE ? CDG_APPLY_ROWSLICE
                     : schedule == CDG_SCHEDULE_AUTO ? CDG_APPLY_AUTO : CDG_APPLY_LEVELS;
     return CDG_OK;
+}
+
+// Whether the next apply of k vectors takes the sweep over W (BF16).
+static bool takes_w(const cdg_prec *M, int k) {
+    if (!M->fold_ok || M->apply_mode == CDG_APPLY_DATAFLOW) return false;
+    if (k > 1 || M->apply_mode == CDG_APPLY_STREAM || M->apply_mode == CDG_APPLY_ROWSLICE) return true;
+    if (M->apply_mode != CDG_APPLY_AUTO) return false;
+    return M->w_asked || (M->fold_after > 0 && (M->napply + k > M->fold_after || M->prev_napply > M->fold_after));
 }
 
 // ---- launch-shape autotuner (no reference counterpart) ---------------------------
@@ -872,20 +890,6 @@ int time_on_stream(cdg_ctx *ctx, hipEvent_t e0, hipEvent_t e1, int reps, F fn, d
     float ms = 0.f;
     CDG_HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
     *ms_out = (double)ms / reps;
-    return CDG_OK;
-}
-
-// Grows the apply's partial-sum storage to the current part_len.
-int prec_part_fit(cdg_ctx *ctx, cdg_prec *M) {
-    const int64_t need = 3 * M->part_len + 2;
-    if (need <= M->part_cap) return CDG_OK;
-    double *np = nullptr;
-    int e = dev_alloc(ctx, (void **)&np, sizeof(double) * (size_t)need);
-    if (e) return e;
-    for (DevMem &m : M->owned)
-        if (m.p == M->d_part) { dev_free(ctx, m.p, m.bytes); m.p = np; m.bytes = sizeof(double) * (size_t)need; }
-    M->d_part = np;
-    M->part_cap = need;
     return CDG_OK;
 }
 
@@ -927,6 +931,15 @@ extern "C" int cdg_prec_tune(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, int32_
     Scratch sc(ctx);
     int e = sc.init((int64_t)M->nrows * n);
     if (e) return e;
+    if (M->apply_mode != CDG_APPLY_FOLDED && M->sweep_ok) {   // the sweep has its shape by a rule: its time only
+        const bool fold = takes_w(M, 1);
+        double ms = 0.0;
+        if (fold) e = sweep_fold(ctx, M, A);
+        if (!e) e = time_on_stream(ctx, sc.e0, sc.e1, reps,
+                                   [&] { return launch_ilu_sweep(ctx, M, A, sc.v, sc.z, (int64_t)M->nrows * n, 1, fold); }, &ms);
+        if (!e && best_ms) *best_ms = ms;
+        return e;
+    }
     // the default first; another shape must beat the best so far by 2 % (the
     // run-to-run spread of one candidate's timing) to replace it
     const ApplyShape def = apply_default(n, prec);
@@ -976,6 +989,7 @@ extern "C" int cdg_mat_tune(cdg_ctx *ctx, cdg_mat *A, int32_t reps, double *best
     std::vector<MvShape> cands{def};
     for (int tg : {128, 256, 384, 540, 768, 1024})
         for (int un : {4, 8, 16}) cands.push_back({tg, un});
+    // (where the flat kernel runs, the loads in flight are its own: the default's number stays)
     std::vector<std::array<int, 2>> seen;
     double best = std::numeric_limits<double>::max();
     const StreamShape keep = A->shape64;
@@ -985,7 +999,7 @@ extern "C" int cdg_mat_tune(cdg_ctx *ctx, cdg_mat *A, int32_t reps, double *best
     for (const MvShape &cand : cands) {
         const int tg = cand.target, un = cand.unroll;
         const StreamShape sh = stream_shape(A->n, 2, tg);
-        if (sh.T == 0) continue;
+        if (sh.T == 0 || (un != def.unroll && mv_flat(ctx, A, sh))) continue;
         const std::array<int, 2> key{sh.T, un};
         if (std::find(seen.begin(), seen.end(), key) != seen.end()) continue;
         seen.push_back(key);
@@ -1081,16 +1095,14 @@ int sweep_fold(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A) {
 // The sweep for k vectors, in the form that M's schedule and history ask for.  Several vectors and
 // the schedules STREAM and ROWSLICE take W where there is one.
 static int prec_sweep(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z, int64_t len, int k) {
-    bool fold = false;
+    const bool fold = takes_w(M, k);
     if (M->fold_ok) {
         M->napply += k;
-        if (k > 1 || M->apply_mode == CDG_APPLY_STREAM || M->apply_mode == CDG_APPLY_ROWSLICE) M->w_asked = 1, fold = true;
-        else if (M->apply_mode == CDG_APPLY_AUTO)
-            fold = M->w_asked || (M->fold_after > 0 && (M->napply > M->fold_after || M->prev_napply > M->fold_after));
-        if (fold) {
-            int e = sweep_fold(ctx, M, A);
-            if (e) return e;
-        }
+        if (k > 1 || M->apply_mode == CDG_APPLY_STREAM || M->apply_mode == CDG_APPLY_ROWSLICE) M->w_asked = 1;
+    }
+    if (fold) {
+        int e = sweep_fold(ctx, M, A);
+        if (e) return e;
     }
     return launch_ilu_sweep(ctx, M, A, v, z, len, k, fold);
 }
@@ -1115,6 +1127,8 @@ static int prec_apply_dev(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const dou
         if (e) return e;
         M->w_ready = 1;
     }
+    int e = prec_part_fit(ctx, M);   // (there, unless the tuned shape has grown)
+    if (e) return e;
     return launch_ilu_apply(ctx, M, A, v, z);
 }
 

@@ -141,7 +141,7 @@ struct cdg_prec {
     int32_t *d_up_ptr = nullptr, *d_up_idx = nullptr, *d_up_col = nullptr, *d_up_blk = nullptr;
     int32_t *d_diag = nullptr;
     int32_t *d_err = nullptr;          // first singular row (factor)
-    double *d_part = nullptr;          // apply partial sums: 3 arrays of part_len doubles
+    double *d_part = nullptr;          // partial sums of the column-slice schedules: 3 arrays of part_len doubles (null: none chosen)
     int64_t part_len = 0;              // nrows * slices * n
     int64_t part_cap = 0;              // doubles allocated at d_part
     // forward levels: rows grouped by level (factor and forward sweep); lower
@@ -235,6 +235,7 @@ int arn_stamp(cdg_ctx *ctx, Arnoldi &A, int i);
 
 // ---- kernel launchers (defined in the .hip files) ----------------------------
 int launch_mv(cdg_ctx *ctx, const cdg_mat *A, const double *x, double *y);
+bool mv_flat(const cdg_ctx *ctx, const cdg_mat *A, const StreamShape &s);
 int launch_ilu_apply(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z);
 int launch_ilu_apply_df(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, const double *v, double *z);
 int df_configure(cdg_ctx *ctx, cdg_prec *M);

@@ -131,7 +131,7 @@ struct cdg_server {
 
 // Device bytes of an ILU(0) preconditioner beyond the matrix: the factor (L,
 // Dinv), the FP32/BF16 copies of the upper blocks, the BF16 variant's FP32
-// work, the block inverse's working slots, the level schedule's partial sums,
+// work, the block inverse's working slots
 // and the sweep's exchange words (nup = nlo: the kind-0 pattern is symmetric).
 static int64_t factor_extra_bytes(int64_t nrows, int64_t nlo, int64_t n, int precision) {
     const int64_t ld = slot_elems((int)n), len = nrows * n;
@@ -140,7 +140,6 @@ static int64_t factor_extra_bytes(int64_t nrows, int64_t nlo, int64_t n, int pre
     if (precision != CDG_FP64) f += es * nlo * ld;               // U copy
     if (precision == CDG_BF16) f += 4 * (nlo + nrows) * ld;      // FP32 factor work
     if (n > 192) f += 8 * nrows * ld;                            // inverse working slots (bound)
-    f += 3 * 8 * nrows * 8 * n;                                  // apply partial sums (<= 8 slices)
     SweepShape sh;                                               // the sweep's exchange words and task records
     if (sweep_shape((int)n, precision, precision == CDG_BF16 ? 4 : 3, 1, 1, 256, &sh))
         for (int64_t k = 1; k <= 8; k *= 8)                      // one vector, and up to eight together

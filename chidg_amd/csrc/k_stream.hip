@@ -502,6 +502,13 @@ StreamShape stream_shape(int n, int V, int target, int tmax) {
     return best;
 }
 
+// Whether the matvec takes the steps of a row's blocks as one sequence (k_mv_flat): fewer steps in a block
+// than loads that should be in flight; with a row alone on its CU the blocks' order matters less than the
+// start (4^3 P1, 64 rows: 5.6 us block by block, 6.7 flat; 216 rows: 8.1 and 6.9)
+bool mv_flat(const cdg_ctx *ctx, const cdg_mat *A, const StreamShape &s) {
+    return A->n * A->n / (2 * s.T) < 8 && 2 * A->nrows > ctx->num_cus;
+}
+
 int launch_mv(cdg_ctx *ctx, const cdg_mat *A, const double *x, double *y) {
     if (A->nrows == 0) return CDG_OK;
     const StreamShape &s = A->shape64;
@@ -510,10 +517,7 @@ int launch_mv(cdg_ctx *ctx, const cdg_mat *A, const double *x, double *y) {
     int chunk = std::max(1, std::min<int>(A->max_row_blocks, (32 * 1024) / (8 * A->n)));
     size_t lds = sizeof(double) * ((size_t)chunk * A->n + (size_t)V * s.T);
     uint64_t *stamp = ctx->hook_stamp ? ctx->hook_stamp + 1 : nullptr;
-    // fewer steps in a block than loads that should be in flight; with a row alone on its CU the blocks'
-    // order matters less than the start (4^3 P1, 64 rows: 5.6 us block by block, 6.7 flat; 216
-    // rows: 8.1 and 6.9)
-    if (A->n * A->n / (V * s.T) < 8 && 2 * A->nrows > ctx->num_cus)
+    if (mv_flat(ctx, A, s))
         hipLaunchKernelGGL(k_mv_flat<8>, dim3(A->nrows), dim3(s.T), lds, ctx->stream, A->blocks, A->ld, A->d_row_ptr,
                            A->d_col, x, y, A->n, s.dc, chunk, ctx->hook_nact, stamp);
     else if (A->mv_unroll == 16)

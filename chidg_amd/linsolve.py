@@ -277,9 +277,9 @@ class _Preconditioner:
 
     def tune(self, A: chidg_matrix, reps: int = 5) -> float:
         """Launch-shape autotuner of the apply on the current factor (after
-        update): keeps the fastest shape for this preconditioner and for later
-        ones of the same block size and precision.  Returns its time per
-        apply in seconds."""
+        update): under 'folded', keeps the fastest shape for this preconditioner
+        and for later ones of the same block size and precision; the sweep has its
+        shape by a rule.  Returns the time per apply in seconds."""
         ms = C.c_double(0.0)
         self.ctx._check(self.ctx.lib.cdg_prec_tune(self.ctx.h, self.h, A.h, int(reps), C.byref(ms)), "cdg_prec_tune")
         return ms.value * 1e-3

@@ -212,18 +212,21 @@ int cdg_prec_destroy(cdg_ctx *ctx, cdg_prec *M);
 #define CDG_SCHEDULE_ROWSLICE 5
 int cdg_prec_set_schedule(cdg_ctx *ctx, cdg_prec *M, int32_t schedule);
 /* Launch-shape autotuner (no reference counterpart).  cdg_prec_tune times the
- * apply of M's current factor (level schedules; after cdg_prec_update) under
- * candidate shapes -- column-slice width, threads per workgroup, 16-byte loads
- * in flight -- `reps` calls each, keeps the fastest for M and remembers it for
- * preconditioners of the same block size and precision created later in the
- * process.  cdg_mat_tune does the same for the matvec (threads, loads in
+ * apply of M's current factor (after cdg_prec_update).  Under
+ * CDG_SCHEDULE_FOLDED, and where rows have too many blocks for the sweep, it
+ * does so under candidate shapes -- column-slice width, threads per workgroup,
+ * 16-byte loads in flight -- `reps` calls each, keeps the fastest for M and
+ * remembers it for preconditioners of the same block size and precision created
+ * later in the process.  The sweep (the other schedules but DATAFLOW, which is
+ * refused) has its shape by a rule: its time is reported and nothing is chosen.
+ * cdg_mat_tune does the same for the matvec (threads, loads in
  * flight; remembered per block size).  *best_ms (may be NULL) receives the
  * chosen shape's time per call.  Results do not depend on the shape beyond
  * rounding (the partial sums regroup). */
 int cdg_prec_tune(cdg_ctx *ctx, cdg_prec *M, const cdg_mat *A, int32_t reps, double *best_ms);
 int cdg_mat_tune(cdg_ctx *ctx, cdg_mat *A, int32_t reps, double *best_ms);
 /* The current shapes: out[4] = {column slices, slice width, threads, loads in
- * flight} for the apply; out[2] = {threads, loads in flight} for the matvec. */
+ * flight} of the apply's column-slice launches; out[2] = {threads, loads in flight} for the matvec. */
 int cdg_prec_launch_shape(const cdg_prec *M, int32_t *out);
 int cdg_mat_launch_shape(const cdg_mat *A, int32_t *out);
 /* Allocation-free apply.  No counterpart in the reference: for callers that
