@@ -151,6 +151,13 @@ static int64_t factor_extra_bytes(int64_t nrows, int64_t nlo, int64_t n, int pre
     return f;
 }
 
+// Device bytes of one FGMRES level's own workspace for k right-hand sides (k_arnoldi.hip): the
+// triangle, rotations and right-hand sides, the partial sums of up to 512 slices.
+static int64_t step_bytes(int64_t m, int64_t len, int64_t k) {
+    const int64_t slices = std::min<int64_t>(512, len / 1024 + 1);
+    return 8 * k * (m * (m + 1) / 2 + 4 * (m + 2) + (4 * m + 6) * (slices + 1) + 32);
+}
+
 extern "C" int cdg_server_footprint(const cdg_request *req, const cdg_fgmres_params *params, int64_t *bytes) {
     if (!req || !params || !bytes) return CDG_ERR_ARG;
     if (req->nx <= 0 || req->ny <= 0 || req->nz <= 0 || req->order < 0 || req->order > 3) return CDG_ERR_ARG;
@@ -165,8 +172,11 @@ extern "C" int cdg_server_footprint(const cdg_request *req, const cdg_fgmres_par
     f += factor_extra_bytes(nrows, nlo, n, req->precision);
     const int64_t m = std::max(1, params->nkrylov);
     const int64_t k = std::max(1, req->nrhs);
-    f += 8 * len * k * (2 * (m + 1) + 6);                        // V, Z, b, x, work vectors per right-hand side
-    if (params->inner_fgmres) f += 8 * len * (2 * (std::max(1, params->inner_nkrylov) + 1) + 4);
+    f += 8 * len * k * (2 * (m + 1) + 6) + step_bytes(m, len, k);   // V, Z, b, x, work vectors per right-hand side
+    if (params->inner_fgmres) {
+        const int64_t mi = std::max(1, params->inner_nkrylov);
+        f += 8 * len * (2 * (mi + 1) + 4) + step_bytes(mi, len, 1);
+    }
     *bytes = f + f / 20 + (64ll << 20);
     return CDG_OK;
 }
@@ -441,8 +451,11 @@ extern "C" int cdg_server_submit_system(cdg_server *s, uint64_t system, const do
         job.home = it->second.home;
         const cdg_mat *A = it->second.A;
         const int64_t len = (int64_t)A->nrows * A->n, m = std::max(1, s->params.nkrylov);
-        job.footprint = 8 * len * (2 * (m + 1) + 8);            // Krylov basis, staging, work vectors
-        if (s->params.inner_fgmres) job.footprint += 8 * len * (2 * (std::max(1, s->params.inner_nkrylov) + 1) + 4);
+        job.footprint = 8 * len * (2 * (m + 1) + 8) + step_bytes(m, len, 1);   // Krylov basis, staging, work vectors
+        if (s->params.inner_fgmres) {
+            const int64_t mi = std::max(1, s->params.inner_nkrylov);
+            job.footprint += 8 * len * (2 * (mi + 1) + 4) + step_bytes(mi, len, 1);
+        }
         job.ticket = s->next_ticket++;
         s->results[job.ticket] = Slot{};
         s->queue.push_back(job);
