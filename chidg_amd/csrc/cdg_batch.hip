@@ -509,7 +509,8 @@ extern "C" int cdg_batch_create(cdg_ctx *ctx, int32_t nsys, cdg_mat *const *A, c
             b0 += A[s]->nnzb;
         }
         {   // row ranges by right-hand-side class: matvecs with 1, 2, 4, 8 vectors per launch,
-            // applies with 2, 4, 8
+            // applies with 2, 4, 8 (systems of one vector go with those of two: their levels run in
+            // the same launch, where a launch of their own would follow; 12 uneven systems 41.8 and 42.1 ms)
             auto cls = [](int k) { return k <= 1 ? 1 : k <= 2 ? 2 : k <= 4 ? 4 : 8; };
             int row = 0;
             for (int s : g.members) {
