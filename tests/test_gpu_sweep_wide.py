@@ -1,5 +1,5 @@
 """The sweep where its levels have more tasks than the GPU has compute units: two levels of a few hundred rows (every
-row of the second half coupled to two of the first), the task shape and the units of several tasks that such
+row of the second half coupled to two or more of the first), the task shape and the units of several tasks that such
 patterns take, with levels that are no multiple of a unit, one and several right-hand sides.  Against the oracle's
 apply; tolerances of the other apply tests, BF16 twice its distance from FP64 (3.5e-3)."""
 import ctypes as C
@@ -23,10 +23,12 @@ def ctx():
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
-@pytest.mark.parametrize("n,half", [(1, 301), (5, 262), (16, 259), (40, 261), (41, 258), (64, 257), (135, 131)])
-def test_two_wide_levels(ctx, n, half, precision):
-    rows = [[(half + (i + d) % half, 0) for d in (0, 1)] + [(i, 0)] for i in range(half)]
-    rows += [sorted(((i - d) % half, 0) for d in (0, 1)) + [(half + i, 0)] for i in range(half)]
+@pytest.mark.parametrize("n,half,links", [(1, 301, 2), (5, 262, 2), (16, 259, 2), (40, 261, 2), (41, 258, 2),
+                                          (64, 257, 2), (135, 131, 2), (22, 300, 7), (32, 260, 7), (42, 260, 6)])
+def test_two_wide_levels(ctx, n, half, links, precision):
+    """(22, 32 and 42 with many links: the most local memory that a unit takes, 76 KB)"""
+    rows = [[(half + (i + d) % half, 0) for d in range(links)] + [(i, 0)] for i in range(half)]
+    rows += [sorted(((i - d) % half, 0) for d in range(links)) + [(half + i, 0)] for i in range(half)]
     p = from_rows(n, rows)
     r = np.random.default_rng(n)
     blocks = r.standard_normal((p.nnzb, n, n)) * (0.2 / np.sqrt(n))
