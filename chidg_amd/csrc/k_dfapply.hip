@@ -124,7 +124,7 @@ template <typename S, typename Acc, int R, int DPF>
 __global__ void __launch_bounds__(kDfMaxThreads, 2) k_df_apply(DfArgs a) {
     constexpr int V = Raw<S>::V;
     typedef typename Raw<S>::T RawT;
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     Acc *xs = reinterpret_cast<Acc *>(smem_raw);          // maxdep * w
     Acc *red = xs + (size_t)a.maxdep * a.w;                // V*T
     __shared__ int sh_task, sh_abort;

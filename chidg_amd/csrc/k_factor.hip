@@ -1199,7 +1199,7 @@ template <typename T, int NR, int UB, bool REPLAY>
 __global__ void __launch_bounds__(kWideThreads) k_fac_ginv(T *__restrict__ D, int64_t ld, T *__restrict__ Wk, int64_t ldw,
                                                    const int32_t *__restrict__ rows, int n,
                                                    int32_t *__restrict__ redo) {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ int32_t flag_sh;
     __shared__ __attribute__((aligned(16))) unsigned char pl_raw[sizeof(PanelLds<T, REPLAY>)];
     PanelLds<T, REPLAY> &pl = *reinterpret_cast<PanelLds<T, REPLAY> *>(pl_raw);
@@ -1579,7 +1579,7 @@ __global__ void __launch_bounds__(kInvThreads) k_fac_pivot(T *__restrict__ D, in
                                                     int32_t *__restrict__ err, int32_t *__restrict__ redo) {
     const int blk = rows[blockIdx.x];
     if (__builtin_amdgcn_readfirstlane(redo[blk]) == 0) return;
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int NP = 16 * ((n + 15) / 16), XPP = NP + 1;
     T *G = reinterpret_cast<T *>(smem_raw);
     T *XP = G + (size_t)NP * 17;

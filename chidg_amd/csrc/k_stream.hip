@@ -308,7 +308,7 @@ struct KSliceArgs {
 template <typename S, typename Acc, int U, int NB, bool P2>
 __global__ void __launch_bounds__(kMaxThreads) k_kslice(KSliceArgs a) {
     constexpr int V = Ld16<S, Acc>::V;
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int T = blockDim.x, tid = threadIdx.x, n = a.n;
     Acc *xs = reinterpret_cast<Acc *>(smem_raw);             // maxdep * w
     Acc *red = xs + (size_t)a.maxdep * a.w;                   // V*T
@@ -376,7 +376,7 @@ template <typename S, typename Acc, int U, int NB>
 __global__ void __launch_bounds__(kMaxThreads) k_dinv_z(const S *__restrict__ D, int64_t ld, VecView t, int Sp,
                                                         int n, int dc, double *__restrict__ z) {
     constexpr int V = Ld16<S, Acc>::V;
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int T = blockDim.x, tid = threadIdx.x, row = blockIdx.x;
     Acc *xs = reinterpret_cast<Acc *>(smem_raw);   // n (n + V*T Acc in all, 16-byte aligned pieces)
     Acc *red = xs + ((n + 3) & ~3);                // V*T
