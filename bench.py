@@ -12,10 +12,10 @@ Inputs are resident in HBM when timing starts.
 ``value`` is the FP32-ILU form's solves/s (ILU factor + apply in FP32, Arnoldi,
 residual and solution in FP64); the plain FP64 form is measured beside it.
 The BF16-stored-ILU form is measured the same way.  The roofline object
-describes the ILU(0) apply (the metric's "ILU apply GB/s") in the schedule a
-long solve settles in (the row-slice schedule: one persistent launch, the sweep
-of csrc/k_sweep.hip over L, U and Dinv), timed with HIP events on the
-library's own stream.  The CPU baseline
+describes the ILU(0) apply (the metric's "ILU apply GB/s") in the form a
+long solve settles in (one persistent launch, the sweep of csrc/k_sweep.hip: over
+L, U and Dinv, or under BF16 storage L, W = Dinv U and Dinv), timed with HIP events
+on the library's own stream.  The CPU baseline
 runs the C oracle (the reference algorithm restated) on the host cores, on the
 same system.
 """
@@ -43,13 +43,13 @@ SEED_Q = 1          # state perturbation
 SEED_B = 1          # right-hand side
 SEED_A = 20261202   # synthetic systems (P3 section, synthetic P2 section)
 HBM_PEAK_GBS = 8000.0
-# The FP32 ILU(0) apply in the row-slice schedule: one call = one launch of
-# k_sweep<float,...>, three tasks per block row (forward, backward, Dinv) and column chunk.
-APPLY_KERNEL = "ILU(0) apply FP32, row-slice schedule: k_sweep<float,1,R,FUSE>, one launch per call"
-# HBM bytes per FP32 row-slice apply call: rocprofv3 FETCH_SIZE (x 2.0) + WRITE_SIZE
+# The FP32 ILU(0) apply: one call = one launch of k_sweep<float,1,5,0>, three tasks per block
+# row (forward, backward, Dinv).
+APPLY_KERNEL = "ILU(0) apply FP32 (sweep): k_sweep<float,1,5,0>, one launch per call"
+# HBM bytes per FP32 apply call: rocprofv3 FETCH_SIZE (x 2.0) + WRITE_SIZE
 # (x 1.0) on the Euler 16^3 P2 system, the factors being what the same counters read for
-# a 512 MiB device copy (985,622 + 21,281 KiB raw per call; the writes are the exchange words).
-APPLY_TRAFFIC_FP32 = 2.040e9
+# a 512 MiB device copy (997,100 + 33,745 KiB raw per call; the writes are the exchange words and z).
+APPLY_TRAFFIC_FP32 = 2.077e9
 
 
 def sig(v, digits=5):
@@ -118,8 +118,9 @@ ITEMSIZE = {"fp64": 8, "fp32": 4, "bf16": 2}
 def measure(args, p, A, b, steps, warmup, kernels=True, precisions=("fp32", "fp64", "bf16")):
     """The FP32-ILU, FP64 and BF16-stored-ILU forms of one system: solves/s
     over ``steps`` timed solves (default schedule), and with ``kernels`` the
-    apply under the level, row-slice, stream and folded schedules, the first
-    row-slice apply's extra time and the matvec, timed on the library stream."""
+    apply (``apply_rowslice_*``: the form a long solve settles in; under BF16 storage
+    also ``apply_levels_*``, the first applies' form, and the time that forming W
+    takes), the folded schedule and the matvec, timed on the library stream."""
     import torch
     from chidg_amd.linsolve import chidg_mv_async, fgmres, precon_ILU0
     ctx = A.ctx
@@ -133,15 +134,6 @@ def measure(args, p, A, b, steps, warmup, kernels=True, precisions=("fp32", "fp6
         x = torch.zeros_like(b)
         for _ in range(warmup):
             ls.solve(A, x, b, M)
-        tune = {}
-        if args.tune:
-            # launch-shape autotuner of the level schedule on the live factor
-            # (setup, outside the timed region)
-            if not warmup:
-                M.update(A)
-            t0 = time.perf_counter()
-            M.tune(A, reps=3)
-            tune = dict(apply_shape=M.launch_shape(), tune_s=time.perf_counter() - t0)
         torch.cuda.synchronize()
         lat = []
         t0 = time.perf_counter()
@@ -157,7 +149,7 @@ def measure(args, p, A, b, steps, warmup, kernels=True, precisions=("fp32", "fp6
                  p50_ms=1e3 * statistics.median(lat), p99_ms=1e3 * float(np.percentile(lat, 99)),
                  niter=st.niter, residual_rel=st.residual_norm / bnorm, true_residual_rel=true_res,
                  t_factor_ms=1e3 * st.t_factor, t_precon_ms=1e3 * st.t_precon, t_mv_ms=1e3 * st.t_mv,
-                 t_dot_ms=1e3 * st.t_dot, t_norm_ms=1e3 * st.t_norm, wall_s=wall, x=x, **tune)
+                 t_dot_ms=1e3 * st.t_dot, t_norm_ms=1e3 * st.t_norm, wall_s=wall, x=x)
         if kernels:
             nbytes = ilu_apply_bytes(p, ITEMSIZE[prec])
             v = b / bnorm
@@ -167,17 +159,16 @@ def measure(args, p, A, b, steps, warmup, kernels=True, precisions=("fp32", "fp6
             # inputs are complete (synchronized above): enqueue without cross-stream waits
             app = lambda: M.apply_async(A, v, z, order=False)   # noqa: E731
             M.update(A)
-            M.set_schedule("levels")
-            t_lv = time_async(ctx, app, args.kreps)
+            if prec == "bf16":                  # (FP64 and FP32: the same launch under both names)
+                M.set_schedule("levels")
+                t_lv = time_async(ctx, app, args.kreps)
+                r.update(apply_levels_ms=1e3 * t_lv, apply_levels_gbs=nbytes / t_lv / 1e9)
             M.set_schedule("rowslice")
             t_first = time_first(ctx, app)
             t_rs = time_async(ctx, app, args.kreps)
-            M.set_schedule("stream")            # the same launch
-            t_st = time_async(ctx, app, args.kreps)
-            r.update(apply_levels_ms=1e3 * t_lv, apply_levels_gbs=nbytes / t_lv / 1e9,
-                     apply_rowslice_ms=1e3 * t_rs, apply_rowslice_gbs=nbytes / t_rs / 1e9,
-                     apply_stream_ms=1e3 * t_st, apply_stream_gbs=nbytes / t_st / 1e9,
-                     rowslice_prep_ms=1e3 * (t_first - t_rs))
+            r.update(apply_rowslice_ms=1e3 * t_rs, apply_rowslice_gbs=nbytes / t_rs / 1e9)
+            if prec == "bf16":
+                r.update(form_w_ms=1e3 * (t_first - t_rs))
             if prec != "bf16" and args.folded:
                 M.update(A)
                 M.set_schedule("folded")
@@ -191,10 +182,8 @@ def measure(args, p, A, b, steps, warmup, kernels=True, precisions=("fp32", "fp6
         out[prec] = r
         log(f"{prec}: {r['solves_per_s']:.2f} solves/s, niter {st.niter}, res {r['residual_rel']:.2e}, "
             f"factor {r['t_factor_ms']:.2f} ms, precon {r['t_precon_ms']:.2f} ms, mv {r['t_mv_ms']:.2f} ms"
-            + (f"; apply levels {r['apply_levels_ms']:.3f} ms ({r['apply_levels_gbs']:.0f} GB/s), row-slice "
-               f"{r['apply_rowslice_ms']:.3f} ms ({r['apply_rowslice_gbs']:.0f} GB/s), stream "
-               f"{r['apply_stream_ms']:.3f} ms ({r['apply_stream_gbs']:.0f} GB/s), prep {r['rowslice_prep_ms']:.2f} "
-               f"ms, mv {r['mv_ms']:.3f} ms ({r['mv_gbs']:.0f} GB/s)" if kernels else ""))
+            + (f"; apply {r['apply_rowslice_ms']:.3f} ms ({r['apply_rowslice_gbs']:.0f} GB/s), "
+               f"mv {r['mv_ms']:.3f} ms ({r['mv_gbs']:.0f} GB/s)" if kernels else ""))
         M.tear_down()
     x64 = out["fp64"].pop("x")
     for prec in precisions:
@@ -256,8 +245,6 @@ def p3_run(args):
         ls = fgmres(nkrylov=30, tol=0.0, rtol=1e-8, inner_fgmres=False)
         x = torch.zeros_like(b)
         ls.solve(A, x, b, M)             # warm-up (allocations)
-        if args.tune:
-            M.tune(A, reps=2)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         ls.solve(A, x, b, M)
@@ -277,10 +264,10 @@ def p3_run(args):
 
 
 def pretune_small(args):
-    """Launch shapes for the request loop's block sizes (P1-P3, FP32 ILU),
-    tuned on 8^3 synthetic systems; the loop's own contexts start from them."""
+    """Matvec launch shapes for the request loop's block sizes (P1-P3), tuned
+    on 8^3 synthetic systems; the loop's own contexts start from them."""
     from chidg_amd import pattern as pt
-    from chidg_amd.linsolve import Context, chidg_matrix, precon_ILU0
+    from chidg_amd.linsolve import Context, chidg_matrix
     ctx = Context(0)
     shapes = {}
     for order in (1, 2, 3):
@@ -289,11 +276,7 @@ def pretune_small(args):
         A = chidg_matrix(p, ctx)
         A.fill_synthetic(SEED_A, 1.0 / np.sqrt(n), 0.1 / np.sqrt(n))
         A.tune(reps=3)
-        M = precon_ILU0("fp32").init(A)
-        M.update(A)
-        M.tune(A, reps=3)
-        shapes[f"P{order}"] = dict(apply=M.launch_shape(), mv=A.launch_shape())
-        M.tear_down()
+        shapes[f"P{order}"] = dict(mv=A.launch_shape())
         A.release()
     ctx.close()
     log(f"pre-tuned launch shapes: {shapes}")
@@ -437,9 +420,8 @@ def cpu_baseline(p, blocks, b, x_gpu):
 
 def profile_workload(name):
     """Short fixed workloads for counter and trace passes (no JSON line):
-    * apply: the FP32 row-slice ILU(0) apply on the Euler 16^3 P2 system, 5
-      times after a first one, then a 512 MiB
-      device copy 3 times (read 512 MiB + write 512 MiB each: the reference
+    * apply: the FP32 ILU(0) apply on the Euler 16^3 P2 system, 5 times after a
+      first one, then a 512 MiB device copy 3 times (read 512 MiB + write 512 MiB each: the reference
       for scaling HBM counters);
     * factor: the ILU(0) factor of the Euler 16^3 P2 system, twice in FP64 and
       twice in FP32, then the seeded synthetic 16^3 P3 system once in FP32 and
@@ -469,7 +451,7 @@ def profile_workload(name):
         for _ in range(5):
             M.apply_async(A, v, z)
         torch.cuda.synchronize()
-        log("apply workload: 5 row-slice applies done")
+        log("apply workload: 5 applies done")
         src = torch.ones(64 * 1024 * 1024, dtype=torch.float64, device="cuda:0")
         dst = torch.empty_like(src)
         for _ in range(3):
@@ -564,7 +546,7 @@ def main():
         parity["gpu_fp64_niter"] = f64["niter"]
         log(f"parity: GPU FP64 {f64['niter']} it vs oracle {parity['oracle_niter']} it, "
             f"x rel {parity['gpu_fp64_x_rel_vs_oracle']:.2e}")
-    # the apply a long solve settles in: the row-slice schedule
+    # the form of the apply a long solve settles in
     t_ap = f32["apply_rowslice_ms"] / 1e3
     gbs = ilu_apply_bytes(p, 4) / t_ap / 1e9
     bf = g.get("bf16")

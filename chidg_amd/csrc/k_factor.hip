@@ -596,9 +596,9 @@ __device__ __forceinline__ bool panel_gj(T *G, int gp, int NP, int n, int k0, in
     return bad;
 }
 
-// 1/x for the pivot chain: v_rcp and Newton steps (within an ulp of the quotient; 3 dependent
-// operations in FP32 and 7 in FP64 instead of the division's 11, which sit on the chain of
-// every pivot step).
+// 1/x for the pivot chain: v_rcp and Newton steps, 3 dependent operations in FP32 and 7 in FP64 instead
+// of the division's 11, which sit on the chain of every pivot step.  In FP64 the last step rounds
+// like the division (a start off by up to 2^-22, 2e8 random x in host FMAs: no difference); in FP32 within an ulp.
 __device__ __forceinline__ float recip(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
     return fmaf(r, fmaf(-x, r, 1.0f), r);
